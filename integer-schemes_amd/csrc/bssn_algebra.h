@@ -26,10 +26,14 @@
 // and may declare `static constexpr bool kEarlyCentres = true` to have the centres of fields
 // not staged yet loaded about a phase before their use (a latency-bound source: the LDS
 // bricks); otherwise each is loaded where it is used.
+// A source for a kernel built to 256 registers declares `static constexpr int kParkSlots = n`
+// with park(slot, x) / parked(slot): the values that live long without being used are kept in
+// its first n slots (LDS, one double per lane and slot) instead of in registers.
 // Out must provide: void put(int f, double rhs)   -- called exactly once per field,
 //                   void metric_done()             -- after the last gt_ij and At_ij put;
 // and may overload out_phase<PH>(Out&), called at the start of phase PH (0 gt, 1 chi, 2 Gt,
-// 3 alpha, 4 beta, 5 At, 6 K, 7 B), to issue loads ahead of its puts.
+// 3 alpha, 4 beta, 5 At, 6 K, 7 B), to issue loads ahead of its puts, or out_prep(Out&, f),
+// called once per field shortly before that field's put.
 #pragma once
 
 #include <type_traits>
@@ -41,6 +45,16 @@ namespace bssn {
 // phase hook of bssn_rhs_point: nothing by default
 template <int PH, class Out>
 __device__ __forceinline__ void out_phase(Out&) {}
+
+// operand hook of bssn_rhs_point (field f will be put soon): nothing by default
+template <class Out>
+__device__ __forceinline__ void out_prep(Out&, int) {}
+
+template <class S, class = void>
+struct ParkSlots : std::integral_constant<int, 0> {};
+template <class S>
+struct ParkSlots<S, std::void_t<decltype(S::kParkSlots)>>
+    : std::integral_constant<int, S::kParkSlots> {};
 
 template <class S, class = void>
 struct EarlyCentres : std::false_type {};
@@ -79,27 +93,63 @@ __device__ __forceinline__ double inverse_sym(const double* g, double* ig) {
   return det;
 }
 
-// At^ij (packed), At_ij At^ij and At_ik gt^kl At_lj from At_ij and gt^ij
+// a0 b0 + a1 b1 + a2 b2 with the roundings fixed: a1 b1 is rounded, the other two products are
+// not. Left to the compiler, which of several products gets fused depends on how often each is
+// used around it, so two kernels that evaluate the same line could differ in the last bit.
+__device__ __forceinline__ double dot3(double a0, double b0, double a1, double b1, double a2,
+                                       double b2) {
+  return __builtin_fma(a2, b2, __builtin_fma(a0, b0, a1 * b1));
+}
+
+// At^ij (packed), At_ij At^ij and At_ik gt^kl At_lj from At_ij and gt^ij. The products
+// gt^ij At_ij (no sum, i != j) occur in two diagonal elements of IA each: dot3 throughout, so
+// that every kernel rounds them alike.
 __device__ __forceinline__ void raise_A(const double* A, const double* ig, double* Aup,
                                         double* AA, double* AkA) {
   double IA[3][3];   // IA[k][j] = gt^kl At_lj
 #pragma unroll
   for (int k = 0; k < 3; ++k)
 #pragma unroll
-    for (int j = 0; j < 3; ++j)
-      IA[k][j] = ig[sym(k, 0)] * A[sym(0, j)] + ig[sym(k, 1)] * A[sym(1, j)] +
-                 ig[sym(k, 2)] * A[sym(2, j)];
+    for (int j = 0; j < 3; ++j) {
+      // (1, 1): the rounded product is gt^xy At_xy, as in (0, 0)
+      const int p = k == 1 && j == 1 ? 1 : 0, r = 1 - p;
+      IA[k][j] = dot3(ig[sym(k, p)], A[sym(p, j)], ig[sym(k, r)], A[sym(r, j)], ig[sym(k, 2)],
+                      A[sym(2, j)]);
+    }
 #pragma unroll
   for (int q = 0; q < 6; ++q) {
     const int i = pi_(q), j = pj_(q);
     Aup[q] = IA[i][0] * ig[sym(0, j)] + IA[i][1] * ig[sym(1, j)] + IA[i][2] * ig[sym(2, j)];
-    if (AkA) AkA[q] = A[sym(i, 0)] * IA[0][j] + A[sym(i, 1)] * IA[1][j] + A[sym(i, 2)] * IA[2][j];
+    if (AkA)
+      AkA[q] = dot3(A[sym(i, 0)], IA[0][j], A[sym(i, 1)], IA[1][j], A[sym(i, 2)], IA[2][j]);
   }
   *AA = contract_sym(Aup, A);
 }
 
 template <bool KO, class Src, class Out>
 __device__ __forceinline__ void bssn_rhs_point(Src& s, const Scal& P, Out& o) {
+  // Values formed early and used late: the gt rates without their Lie terms (gt phase to At
+  // phase), the trace-free curvature part of the At rates (alpha to At), the advection and
+  // Kreiss-Oliger terms of Gt (Gt to the end); slots past the source's are registers.
+  constexpr int PK = ParkSlots<Src>::value;
+  enum : int { P_RG = 0, P_RA = 6, P_ADV = 12, P_KOG = 15, P_N = 18 };
+  double held[P_N];
+  auto keep = [&](int i, double x) {
+    if constexpr (PK > 0) {
+      if (i < PK) {
+        s.park(i, x);
+        return;
+      }
+    }
+    held[i] = x;
+  };
+  auto kept = [&](int i) -> double {
+    if constexpr (PK > 0) {
+      if (i < PK) return s.parked(i);
+    }
+    return held[i];
+  };
+
   // ---------------------------------------------------------------- metric and shift centres
   double g[6], ig[6], b[3];
 #pragma unroll
@@ -113,7 +163,6 @@ __device__ __forceinline__ void bssn_rhs_point(Src& s, const Scal& P, Out& o) {
   // ---------------------------------------------------------------- gt_ij: Christoffels, Rt
   out_phase<0>(o);
   double Rt[6];        // accumulates the Ricci tensor
-  double rg[6];        // gt right-hand sides (advection + KO so far)
   double C2[3][6], CalGt[3];
   // Early centres: the centre values of fields not staged yet are loaded about a phase before
   // their use, so their latency hides behind work (LDS bricks at 256^3 FD4/KO6: RK4 step
@@ -138,7 +187,15 @@ __device__ __forceinline__ void bssn_rhs_point(Src& s, const Scal& P, Out& o) {
       Rt[q] = -0.5 * lapg;
       double r = b[0] * dg[0][q] + b[1] * dg[1][q] + b[2] * dg[2][q];
       if (KO) r += s.ko();
-      rg[q] = pin(r);
+      keep(P_RG + q, pin(r));
+    }
+    // the Ricci tensor is the widest point: the metric and the shift, which it does not use,
+    // wait in slots whose values are formed later
+    if constexpr (PK > 0) {
+#pragma unroll
+      for (int q = 0; q < 6; ++q) keep(P_RA + q, g[q]);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) keep(P_ADV + i, b[i]);
     }
     double C1[3][6];   // Gamma_k(ij), first index lowered
 #pragma unroll
@@ -194,20 +251,29 @@ __device__ __forceinline__ void bssn_rhs_point(Src& s, const Scal& P, Out& o) {
 #pragma unroll
   for (int m = 0; m < 3; ++m) BSSN_PIN(CalGt[m]);
 
-  // At^ij from the At centres, for the two contractions needed before the Christoffels die:
-  // Gamma^i_jk At^jk and At_ij At^ij.
-  double CA[3], AA;
-  {
-    if (!EC) {
+  if constexpr (PK > 0) {
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int p = 0; p < 6; ++p) Acen[p] = s.center(AT0 + p);
-    }
+    for (int q = 0; q < 6; ++q) g[q] = kept(P_RA + q);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) b[i] = kept(P_ADV + i);
+  }
+  // At^ij from the At centres, for the two contractions needed before the Christoffels die:
+  // Gamma^i_jk At^jk and At_ij At^ij. With parked values (several waves per SIMD) the centres
+  // are loaded here and contracted after the chi phase, which hides their latency.
+  double CA[3], AA;
+  if (!EC) {
+#pragma unroll
+    for (int p = 0; p < 6; ++p) Acen[p] = s.center(AT0 + p);
+  }
+  auto contract_At = [&]() {
     double Aup[6];
     raise_A(Acen, ig, Aup, &AA, nullptr);
 #pragma unroll
     for (int i = 0; i < 3; ++i) CA[i] = pin(contract_sym(C2[i], Aup));
     BSSN_PIN(AA);
-  }
+  };
+  if constexpr (PK == 0) contract_At();
 
   // ---------------------------------------------------------------- chi: Ricci chi part
   out_phase<1>(o);
@@ -245,8 +311,8 @@ __device__ __forceinline__ void bssn_rhs_point(Src& s, const Scal& P, Out& o) {
 
   // ---------------------------------------------------------------- Gt^k: d_(i Gt_j) term
   out_phase<2>(o);
+  if constexpr (PK > 0) contract_At();
   double K = EC ? s.center(KTR) : 0.0;
-  double advGt[3], koGt[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     s.stage(GTI0 + k);
@@ -258,8 +324,8 @@ __device__ __forceinline__ void bssn_rhs_point(Src& s, const Scal& P, Out& o) {
       const int i = pi_(q), j = pj_(q);
       Rt[q] += 0.5 * (g[sym(k, i)] * dG[j] + g[sym(k, j)] * dG[i]);
     }
-    advGt[k] = pin(b[0] * dG[0] + b[1] * dG[1] + b[2] * dG[2]);
-    koGt[k] = KO ? s.ko() : 0.0;
+    keep(P_ADV + k, pin(b[0] * dG[0] + b[1] * dG[1] + b[2] * dG[2]));
+    keep(P_KOG + k, KO ? s.ko() : 0.0);
   }
   // R_ij is complete from here on.
 
@@ -271,8 +337,9 @@ __device__ __forceinline__ void bssn_rhs_point(Src& s, const Scal& P, Out& o) {
 #pragma unroll
     for (int i = 0; i < 3; ++i) Bcen[i] = s.center(BB0 + i);
   }
-  double al, dal[3], rGt[3], rK, rA[6];
+  double al, dal[3], rGt[3], rK;
   {
+    out_prep(o, ALPHA);
     s.stage(ALPHA);
     al = s.val();
 #pragma unroll
@@ -297,7 +364,7 @@ __device__ __forceinline__ void bssn_rhs_point(Src& s, const Scal& P, Out& o) {
     for (int q = 0; q < 6; ++q) X[q] = al * Rt[q] - DD[q];
     const double trX3 = contract_sym(ig, X) * (1.0 / 3.0);
 #pragma unroll
-    for (int q = 0; q < 6; ++q) rA[q] = pin(chi * (X[q] - g[q] * trX3));
+    for (int q = 0; q < 6; ++q) keep(P_RA + q, pin(chi * (X[q] - g[q] * trX3)));
     rK = pin(-chi * contract_sym(ig, DD));
     // Hamiltonian constraint and its damping of chi (CAHD)
     const double ham = chi * Rs - AA + (2.0 / 3.0) * K * K;
@@ -309,7 +376,7 @@ __device__ __forceinline__ void bssn_rhs_point(Src& s, const Scal& P, Out& o) {
     if (KO) ra += s.ko();
     o.put(ALPHA, ra);
 #pragma unroll
-    for (int i = 0; i < 3; ++i) rGt[i] = pin(advGt[i] + 2.0 * al * CA[i]);
+    for (int i = 0; i < 3; ++i) rGt[i] = pin(kept(P_ADV + i) + 2.0 * al * CA[i]);
   }
   // The Christoffels and the Ricci tensor are dead from here on.
 
@@ -320,6 +387,9 @@ __device__ __forceinline__ void bssn_rhs_point(Src& s, const Scal& P, Out& o) {
     const double Bf = 0.75 * (P.lamf[0] + P.lamf[1] * al);
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
+      out_prep(o, BETA0 + i);
+      if (i == 2) out_prep(o, CHI);
+      if (!EC && PK > 0) Bcen[i] = s.center(BB0 + i);   // several waves per SIMD: ahead of use
       s.stage(BETA0 + i);
 #pragma unroll
       for (int a = 0; a < 3; ++a) db[a][i] = s.d1(a);
@@ -332,7 +402,7 @@ __device__ __forceinline__ void bssn_rhs_point(Src& s, const Scal& P, Out& o) {
       for (int m = 0; m < 3; ++m)
         rGt[m] += (1.0 / 3.0) * (ig[sym(m, 0)] * d2b[sym(0, i)] + ig[sym(m, 1)] * d2b[sym(1, i)] +
                                  ig[sym(m, 2)] * d2b[sym(2, i)]);
-      if (!EC) Bcen[i] = s.center(BB0 + i);
+      if (!EC && PK == 0) Bcen[i] = s.center(BB0 + i);
       double rb = Bf * Bcen[i] +
                   P.lam[1] * (b[0] * db[0][i] + b[1] * db[1][i] + b[2] * db[2][i]);
       if (KO) rb += s.ko();
@@ -357,7 +427,14 @@ __device__ __forceinline__ void bssn_rhs_point(Src& s, const Scal& P, Out& o) {
       A[q] = s.val();
       double r = b[0] * s.d1(0) + b[1] * s.d1(1) + b[2] * s.d1(2);
       if (KO) r += s.ko();
-      rA[q] += r;
+      keep(P_RA + q, kept(P_RA + q) + r);
+    }
+    // operands of the At and gt puts two pairs ahead (all twelve at once would add 48 registers
+    // to the second widest point)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      out_prep(o, AT0 + q);
+      out_prep(o, GT0 + q);
     }
     double Aup[6], AA2, AkA[6];
     raise_A(A, ig, Aup, &AA2, AkA);
@@ -375,14 +452,18 @@ __device__ __forceinline__ void bssn_rhs_point(Src& s, const Scal& P, Out& o) {
 #pragma unroll
     for (int q = 0; q < 6; ++q) {
       const int i = pi_(q), j = pj_(q);
+      if (q < 4) {
+        out_prep(o, AT0 + q + 2);
+        out_prep(o, GT0 + q + 2);
+      }
       double lie = 0.0, lieg = 0.0;
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
         lie += A[sym(i, k)] * db[j][k] + A[sym(k, j)] * db[i][k];
         lieg += g[sym(i, k)] * db[j][k] + g[sym(k, j)] * db[i][k];
       }
-      o.put(AT0 + q, rA[q] + lie - (2.0 / 3.0) * A[q] * divb + al * (K * A[q] - 2.0 * AkA[q]));
-      o.put(GT0 + q, rg[q] + lieg - (2.0 / 3.0) * g[q] * divb - 2.0 * al * A[q]);
+      o.put(AT0 + q, kept(P_RA + q) + lie - (2.0 / 3.0) * A[q] * divb + al * (K * A[q] - 2.0 * AkA[q]));
+      o.put(GT0 + q, kept(P_RG + q) + lieg - (2.0 / 3.0) * g[q] * divb - 2.0 * al * A[q]);
     }
     o.metric_done();
   }
@@ -390,6 +471,7 @@ __device__ __forceinline__ void bssn_rhs_point(Src& s, const Scal& P, Out& o) {
   // ---------------------------------------------------------------- K
   out_phase<6>(o);
   {
+    out_prep(o, KTR);
     s.stage(KTR);
     double dK[3];
 #pragma unroll
@@ -407,12 +489,14 @@ __device__ __forceinline__ void bssn_rhs_point(Src& s, const Scal& P, Out& o) {
   out_phase<7>(o);
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
+    out_prep(o, BB0 + i);
+    out_prep(o, GTI0 + i);
     s.stage(BB0 + i);
     double r = rGt[i] - P.eta * s.val() +
-               P.lam[2] * (b[0] * s.d1(0) + b[1] * s.d1(1) + b[2] * s.d1(2)) - P.lam[3] * advGt[i];
+               P.lam[2] * (b[0] * s.d1(0) + b[1] * s.d1(1) + b[2] * s.d1(2)) - P.lam[3] * kept(P_ADV + i);
     if (KO) r += s.ko();
     o.put(BB0 + i, r);
-    o.put(GTI0 + i, rGt[i] + koGt[i]);
+    o.put(GTI0 + i, rGt[i] + kept(P_KOG + i));
   }
 }
 

@@ -20,6 +20,7 @@
 
 #include "bssn_algebra.h"
 #include "bssn_brick.h"
+#include "bssn_group.h"
 #include "bssn_kernels.h"
 #include "bssn_params.h"
 #include "bssn_stage.h"
@@ -45,12 +46,41 @@ void k_fused(StageArgs args, Dims d, Scales w, Scal sc) {
   bssn_rhs_point<KO>(src, with_ssl(sc, args.tdev, args.toff), out);
 }
 
+// The same on bricks shared by four waves, two waves per SIMD (bssn_group.h); equal results.
+template <int ORD, bool KO, int MODE, int KIND, bool SDEV>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(2, 2)))
+void k_fused_group(StageArgs args, Dims d, Scales w, Scal sc) {
+  using G = GroupGeo<ORD, KO>;
+  static_assert(G::NT == 256, "launch bounds");
+  __shared__ double mem[G::LDS_DOUBLES];
+  int ox, oy, oz;
+  if (!brick_origin<G>(d, &ox, &oy, &oz)) return;
+  const int t = (int)threadIdx.x;
+  if constexpr (SDEV) args_from_pack<ORD>(args, w, sc);
+  GroupSrc<ORD, KO, MODE> src(mem, args.Yin, w, d, ox, oy, oz, t);
+  StageOut<KIND, true> out(args, d.P, src.gc, lane_valid<G>(d, ox, oy, oz, t), true);
+  bssn_rhs_point<KO>(src, with_ssl(sc, args.tdev, args.toff), out);
+}
+
+// A grid whose wave-private bricks all fit the chip at once, one per SIMD (4 x 256), is one
+// wave's latency long either way, and the wave-private form's is the shorter (no barriers, more
+// registers): FD4 RK4 step at 24^3 / 32^3 / 40^3 (1000 bricks) 115 / 127 / 155 us against 135 /
+// 141 / 192 us. Past it the shared bricks win: 48^3 (1728) 271 against 213, 64^3 539 against
+// 430, 128^3 4.39 against 3.20 ms.
+constexpr unsigned kWaveBricks = 4 * 256;
+
 template <int ORD, bool KO, int MODE, int KIND, bool SDEV>
 static hipError_t launch_fused_t(const StageArgs& a, const Dims& d, const Scales& w,
                                  const Scal& sc, hipStream_t st) {
-  using G = Geo<ORD, KO>;
-  hipLaunchKernelGGL((k_fused<ORD, KO, MODE, KIND, SDEV>), dim3(brick_blocks<G>(d)),
-                     dim3(G::NT), 0, st, a, d, w, sc);
+  using W = Geo<ORD, KO>;
+  using G = GroupGeo<ORD, KO>;
+  if (brick_blocks<W>(d) <= kWaveBricks)
+    hipLaunchKernelGGL((k_fused<ORD, KO, MODE, KIND, SDEV>), dim3(brick_blocks<W>(d)),
+                       dim3(W::NT), 0, st, a, d, w, sc);
+  else
+    hipLaunchKernelGGL((k_fused_group<ORD, KO, MODE, KIND, SDEV>), dim3(brick_blocks<G>(d)),
+                       dim3(G::NT), 0, st, a, d, w, sc);
   return hipGetLastError();
 }
 

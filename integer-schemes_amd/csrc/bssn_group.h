@@ -1,0 +1,137 @@
+// Bricks shared by the waves of a workgroup, for the fused kernels.
+//
+// One workgroup is four waves owning a 4 x 4 x 16 brick of output points (one point per lane, z
+// fastest). The four waves stage one field at a time into a common LDS box (the brick plus H on
+// every side), so a point costs about half the staged cells of a wave-private 4 x 4 x 4 brick
+// (FD order 4 with KO: 5.9 instead of 8.5 loads per point for the fields with mixed derivatives,
+// 4.4 instead of 5.5 for the others), and its rows are runs of 16 to 22 doubles instead of 4 to
+// 10, both in the loads and in the stores.
+//
+// What bounds the fused stage kernels is unhidden latency: at one wave per SIMD (the
+// wave-private form needs 374-438 registers) the 256^3 FD4 RK4 step takes 37.4 ms, of which 21.4
+// ms remain with every staging load, write-back operand and store left out. Two waves per SIMD
+// cover each other, but must fit 256 registers:
+//   * fewer staged cells per lane (6 instead of 9) and one in-flight set of them;
+//   * the write-back operands of a field are loaded shortly before its put (StageOut NEAR);
+//   * 18 long-lived values per point are parked in LDS (bssn_rhs_point's keep/kept), which the
+//     shared box leaves room for: 2 boxes of 17.2 KB and 36 KB of slots, two workgroups per CU.
+// 16-22 registers per lane still spill. Measured at 256^3, FD4 with KO 6, RK4 step / bare RHS:
+// 37.37 / 5.96 -> 26.0 / 4.64 ms; other shapes 4x8x8 27.8 / 4.65, 2x8x16 27.0 / 4.86,
+// 8x8x8 29.0 / 5.06, 4x8x16 27.1 / 5.00, 8x4x16 27.3 / 5.12, 8x2x16 28.3 / 4.90,
+// 4x4x8 (two waves) 31.5 / 4.84 ms.
+//
+// The boxes alternate, so one barrier per field is enough: the box written for field i was last
+// read for field i - 2, and a wave passes the barrier of field i - 1 only after those reads.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "bssn_brick.h"
+
+namespace bssn {
+
+template <int ORD, bool KO>
+struct GroupGeo {
+  static constexpr int R = Coef<ORD>::R;                  // FD reach
+  static constexpr int RK = KO ? Coef<ORD>::RK : 0;       // KO reach
+  static constexpr int H = R > RK ? R : RK;               // box halo
+  static constexpr int BX = 4, BY = 4, BZ = 16;           // brick
+  static constexpr int NT = BX * BY * BZ;                 // lanes (four waves)
+  static constexpr int NX = BX + 2 * H, NY = BY + 2 * H, NZ = BZ + 2 * H;   // box extents
+  // dense rows and planes: the 16 lanes of one LDS access phase read one z row of the brick, 16
+  // distinct bank pairs whatever the pitch
+  static constexpr int SY = NZ, SX = NY * NZ, VOL = NX * SX;
+  static_assert(NX < 32 && NY < 32 && NZ < 32, "box coordinates are packed in 5 bits");
+  static constexpr int NCORE = BX * BY * BZ;
+  static constexpr int NFACE = 2 * H * (BY * BZ + BX * BZ + BX * BY);
+  static constexpr int NEDGE = 4 * R * R * (BX + BY + BZ);
+  __host__ __device__ static constexpr int lx(int t) { return t / (BY * BZ); }
+  __host__ __device__ static constexpr int ly(int t) { return (t / BZ) % BY; }
+  __host__ __device__ static constexpr int lz(int t) { return t % BZ; }
+  static constexpr int NCELL = NCORE + NFACE + NEDGE;
+  static constexpr int PER = (NCELL + NT - 1) / NT;       // staged cells per lane
+  static constexpr int PER_FACES = (NCORE + NFACE + NT - 1) / NT;
+  // parked values per point: all 18, or as many as let two workgroups share a CU's 160 KB of LDS
+  // (13 with the wider boxes of FD orders 6 and 8)
+  static constexpr int ROOM = (80 * 1024 / 8 - 2 * VOL) / NT;
+  static constexpr int SLOTS = ROOM < 18 ? ROOM : 18;
+  static_assert(SLOTS >= 12, "the gt and At rates must fit");
+  static constexpr int LDS_DOUBLES = 2 * VOL + SLOTS * NT;
+};
+
+// Barrier of the workgroup that orders its LDS accesses (global loads and stores stay in
+// flight across it).
+__device__ __forceinline__ void group_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Source of fields and derivatives for bssn_rhs_point over shared boxes: as WaveSrc with one
+// field in flight, with a workgroup barrier where WaveSrc relies on a wave's LDS order. Every
+// lane of the workgroup must run the whole stage sequence (lanes without a point of their own
+// stage cells for the others).
+template <int ORD, bool KO, int MODE>
+struct GroupSrc : BoxStencil<GroupGeo<ORD, KO>, Coef<ORD>> {
+  using G = GroupGeo<ORD, KO>;
+  using Box = BoxStencil<G, Coef<ORD>>;
+  using Box::c;
+  using Box::lds;
+  double* boxes;        // two boxes
+  double* slots;        // this lane's parked values, NT apart
+  const double* F;
+  long P;
+  int off[G::PER];      // grid offsets of this lane's staged cells
+  int cel[G::PER];      // box indices of this lane's staged cells
+  double pf[G::PER];    // the next field's cells, in flight
+  long gc;              // flat index of the lane's point (clamped into the grid)
+  static constexpr int kParkSlots = G::SLOTS;
+
+  __device__ __forceinline__ GroupSrc(double* mem, const double* F_, const Scales& sc_,
+                                      const Dims& d, int ox, int oy, int oz, int t)
+      : Box(mem, sc_), boxes(mem), slots(mem + 2 * G::VOL + t), F(F_), P(d.P) {
+    c = (G::lx(t) + G::H) * G::SX + (G::ly(t) + G::H) * G::SY + (G::lz(t) + G::H);
+    gc = lane_point<G>(d, ox, oy, oz, t);
+    const int o[3] = {ox, oy, oz};
+#pragma unroll
+    for (int k = 0; k < G::PER; ++k) {
+      const int e = kCells<G>.c[t + k * G::NT];
+      const int cc[3] = {e & 31, (e >> 5) & 31, (e >> 10) & 31};
+      cel[k] = cc[0] * G::SX + cc[1] * G::SY + cc[2];
+      int g[3];
+#pragma unroll
+      for (int a = 0; a < 3; ++a) g[a] = map_axis<MODE>(o[a] + cc[a] - G::H, d.S[a], d.ng);
+      off[k] = (g[0] * d.S[1] + g[1]) * d.S[2] + g[2];
+    }
+    fetch(RhsOrder::at(0));
+  }
+
+  __device__ __forceinline__ static int cells(int f) {
+    return needs_edges(f) ? G::PER : G::PER_FACES;
+  }
+
+  __device__ __forceinline__ void fetch(int f) {
+    const double* u = F + (long)f * P;
+    const int n = cells(f);
+#pragma unroll
+    for (int k = 0; k < G::PER; ++k)
+      if (k < n) pf[k] = u[off[k]];
+    __builtin_amdgcn_sched_barrier(0);   // keep the loads here, ahead of the work they overlap
+  }
+
+  __device__ __forceinline__ void stage(int f) {
+    const int at = RhsOrder::pos(f), n = cells(f);
+    lds = boxes + (at & 1) * G::VOL;
+#pragma unroll
+    for (int k = 0; k < G::PER; ++k)
+      if (k < n) lds[cel[k]] = pf[k];
+    group_barrier();
+    if (at + 1 < RhsOrder::N) fetch(RhsOrder::at(at + 1));
+  }
+
+  __device__ __forceinline__ double center(int f) const { return F[(long)f * P + gc]; }
+  __device__ __forceinline__ void park(int i, double x) { slots[i * G::NT] = x; }
+  __device__ __forceinline__ double parked(int i) const { return slots[i * G::NT]; }
+};
+
+}  // namespace bssn

@@ -83,7 +83,10 @@ constexpr int fused_depth() {
 // The write-back kind is a template parameter: each launch runs the code of its own kind only
 // (a runtime switch over all kinds made the stage kernel half again as large).
 // RK2 and RK3 share their code (c0 differs); KIND_RK3 launches StageOut<KIND_RK2>.
-template <int KIND>
+// NEAR: the operands of a field are loaded when bssn_rhs_point announces its put (out_prep),
+// for the kernels whose other waves hide what is left of the latency and whose 256 registers
+// cannot hold them longer; else BSSN_WB_LEAD phases ahead.
+template <int KIND, bool NEAR = false>
 struct StageOut {
   const StageArgs& A;
   long P, gp;
@@ -130,7 +133,7 @@ struct StageOut {
   // called by bssn_rhs_point at the start of phase PH
   template <int PH>
   __device__ __forceinline__ void phase() {
-    if (!deferred) return;
+    if (NEAR || !deferred) return;
 #pragma unroll
     for (int f = 0; f < BSSN_NF; ++f)
       if (load_phase(f) == PH) load(f);
@@ -188,11 +191,16 @@ struct StageOut {
   }
 };
 
-// bssn_rhs_point's phase hook for the stage write-back (more specialised than its generic,
-// empty hook)
-template <int PH, int KIND>
-__device__ __forceinline__ void out_phase(StageOut<KIND>& o) {
+// bssn_rhs_point's hooks for the stage write-back (more specialised than its generic, empty
+// ones)
+template <int PH, int KIND, bool NEAR>
+__device__ __forceinline__ void out_phase(StageOut<KIND, NEAR>& o) {
   o.template phase<PH>();
+}
+template <int KIND>
+__device__ __forceinline__ void out_prep(StageOut<KIND, true>& o, int f) {
+  o.load(f);
+  __builtin_amdgcn_sched_barrier(0);   // keep the loads here, ahead of the work they overlap
 }
 
 // Call fn(std::integral_constant<int, K>) with K the template kind of the runtime stage kind

@@ -1,0 +1,114 @@
+"""GPU: the fused kernels on bricks shared by four waves (grids of more than 1024 wave-private
+bricks), against the oracle and against the wave-private kernels of the batched form, at extents
+one short of, on and one past the 4 x 4 x 16 brick, thin axes, and on both sides of the rule that
+picks the kernel.
+
+Tolerance 1e-12 normwise per field. The states are sinusoids of 12 to 24 points per wave and
+amplitude 0.05 at h ~ 0.1, so second derivatives are ~1 and their rounding error, eps times the
+sum of the stencil's weights over h^2 (order 8: 2.2e-16 x 6.5 / 0.0081), is below 2e-13 of the
+rates they enter; every other term is smaller.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as O
+from conftest import gpu_available, normwise
+
+from bssn3d_hip.batch import Block, BlockBatch
+from bssn3d_hip.evolve import BSSNEvolution
+from bssn3d_hip.grid import Grid
+from bssn3d_hip.rhs import rhs_into
+from bssn3d_hip.state import PhysicsParams, scalars
+
+pytestmark = [pytest.mark.gpu,
+              pytest.mark.skipif(not gpu_available(), reason="needs a HIP device")]
+
+TOL = 1e-12
+DEV = "cuda:0"
+H3 = (0.1, 0.11, 0.09)
+P = PhysicsParams()
+
+
+def waves(shape, seed, periodic=False, ng=0):
+    """24 sinusoids, a whole number of waves per interior axis where periodic."""
+    rng = np.random.default_rng(seed)
+    F = np.zeros((24,) + tuple(shape))
+    for f in range(24):
+        arg = rng.uniform(0, 6)
+        for a, n in enumerate(shape):
+            m = n - 2 * ng
+            cycles = max(1, m // 16) if periodic else m / rng.uniform(12, 24)
+            x = 2 * np.pi * cycles * (np.arange(n) - ng) / m
+            arg = arg + rng.choice([-1, 1]) * x.reshape([-1 if b == a else 1 for b in range(3)])
+        F[f] = 0.05 * np.sin(arg)
+    for f in (0, 1, 3, 6, 8):
+        F[f] += 1.0
+    return F
+
+
+def bricks(shape):
+    return int(np.prod([(n + 3) // 4 for n in shape]))
+
+
+@pytest.mark.parametrize("shape", [(40, 40, 40), (36, 44, 47), (37, 45, 48), (35, 43, 49),
+                                   (2, 70, 260), (41, 3, 433), (85, 90, 9)])
+@pytest.mark.parametrize("order", [4, 6, 8])
+@pytest.mark.parametrize("ko", [0.0, 0.1])
+def test_rhs(shape, order, ko):
+    print(f"[case] rhs {shape} order {order} ko {ko}", flush=True)
+    assert (bricks(shape) > 1024) == (shape != (40, 40, 40))
+    F = waves(shape, seed=sum(shape) + order)
+    S16 = scalars(P, *H3, 0.02, 0.4)
+    Fd = torch.from_numpy(F).to(DEV)
+    out = torch.empty_like(Fd)
+    rhs_into(Fd, out, S16, order, ko)
+    err = normwise(out.cpu().numpy(), O.rhs(F, S16, order, ko_sigma=ko))
+    assert err.max() < TOL, err
+
+
+@pytest.mark.parametrize("interior,order,integrator,bc",
+                         [((41, 45, 48), 4, "rk4", "periodic"),
+                          ((40, 43, 49), 4, "rk4_2_2", "periodic"),
+                          ((44, 42, 47), 6, "rk4", "none"),
+                          ((42, 41, 65), 6, "rk4_2_2", "periodic"),
+                          ((45, 44, 47), 8, "rk4", "periodic")])
+def test_steps(interior, order, integrator, bc):
+    print(f"[case] {integrator} {interior} order {order} {bc}", flush=True)
+    ng = 3 if order == 4 else 4
+    grid = Grid(*interior, *H3, ng=ng)
+    F = waves(grid.shape, seed=order, periodic=True, ng=ng)
+    dt = 0.02
+    evo = BSSNEvolution(grid, P, order=order, ko_sigma=0.1, bc=bc, integrator=integrator)
+    got = evo.evolve(torch.from_numpy(F).to(DEV), dt, 2, t0=0.1).data.cpu().numpy()
+    S16 = scalars(P, *H3, dt, 0.1)
+    if bc == "periodic":
+        ref = O.periodic_sync(O.evolve(F, S16, dt, 2, t0=0.1, integrator=integrator, order=order,
+                                       ko_sigma=0.1, ng=ng), ng)
+    else:
+        ref = O.evolve(F, S16, dt, 2, t0=0.1, integrator=integrator, order=order, ko_sigma=0.1,
+                       ng=ng, periodic=False)
+    err = normwise(got, ref)
+    assert err.max() < TOL, err
+
+
+@pytest.mark.parametrize("n", [(42, 39, 50), (34, 61, 64)])
+def test_equals_batched_form(n):
+    """One block through the batched kernels: the same bits."""
+    print(f"[case] batch {n}", flush=True)
+    batch = BlockBatch([Block(n=n, h=H3)], ng=3, device=DEV)
+    U = batch.empty_pool()
+    batch.view(U, 0).copy_(torch.from_numpy(waves([v + 6 for v in n], 7, True, 3)))
+    F = batch.view(U, 0).clone()
+    out, one = torch.empty_like(U), torch.empty_like(F)
+    batch.rhs_into(U, out, P, 0.02, order=4, ko_sigma=0.1)
+    S16 = scalars(P, *H3, 0.02, 0.0)
+    S16[3] = H3[0]
+    rhs_into(F, one, S16, 4, 0.1)
+    assert torch.equal(batch.view(out, 0), one)
+    evo = BSSNEvolution(Grid(*n, *H3, ng=3), P, order=4, ko_sigma=0.1)
+    evo.step_(F, 0.0, 0.02)
+    batch.step_(U, 0.0, 0.02, P, order=4, ko_sigma=0.1, bc="periodic")
+    assert torch.equal(batch.view(U, 0), F)
