@@ -68,14 +68,17 @@ void k_fused_group(StageArgs args, Dims d, Scales w, Scal sc) {
 // registers): FD4 RK4 step at 24^3 / 32^3 / 40^3 (1000 bricks) 115 / 127 / 155 us against 135 /
 // 141 / 192 us. Past it the shared bricks win: 48^3 (1728) 271 against 213, 64^3 539 against
 // 430, 128^3 4.39 against 3.20 ms.
+// The shared form addresses a field by 32-bit byte offsets, so fields of 4 GiB and more (a state
+// of 103 GB: only the bare RHS fits the card) take the wave-private form too.
 constexpr unsigned kWaveBricks = 4 * 256;
+constexpr long kGroupPoints = 1L << 29;
 
 template <int ORD, bool KO, int MODE, int KIND, bool SDEV>
 static hipError_t launch_fused_t(const StageArgs& a, const Dims& d, const Scales& w,
                                  const Scal& sc, hipStream_t st) {
   using W = Geo<ORD, KO>;
   using G = GroupGeo<ORD, KO>;
-  if (brick_blocks<W>(d) <= kWaveBricks)
+  if (brick_blocks<W>(d) <= kWaveBricks || d.P >= kGroupPoints)
     hipLaunchKernelGGL((k_fused<ORD, KO, MODE, KIND, SDEV>), dim3(brick_blocks<W>(d)),
                        dim3(W::NT), 0, st, a, d, w, sc);
   else

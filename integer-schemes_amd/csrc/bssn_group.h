@@ -15,10 +15,13 @@
 //   * the write-back operands of a field are loaded shortly before its put (StageOut NEAR);
 //   * 18 long-lived values per point are parked in LDS (bssn_rhs_point's keep/kept), which the
 //     shared box leaves room for: 2 boxes of 17.2 KB and 36 KB of slots, two workgroups per CU.
-// 16-22 registers per lane still spill. Measured at 256^3, FD4 with KO 6, RK4 step / bare RHS:
-// 37.37 / 5.96 -> 26.0 / 4.64 ms; other shapes 4x8x8 27.8 / 4.65, 2x8x16 27.0 / 4.86,
-// 8x8x8 29.0 / 5.06, 4x8x16 27.1 / 5.00, 8x4x16 27.3 / 5.12, 8x2x16 28.3 / 4.90,
-// 4x4x8 (two waves) 31.5 / 4.84 ms.
+//   * fields are addressed by 32-bit byte offsets from their uniform base (fields below 4 GiB):
+//     with 64-bit indices the address pairs of 9 fields lived, spilled, from the first loads to
+//     the last stores, 1.1 GB of scratch written per stage (step 26.0, bare RHS 4.81 ms).
+// Measured at 256^3, FD4 with KO 6, RK4 step / bare RHS: wave-private 37.37 / 5.96, shared 24.1 /
+// 4.52 ms (FD order 4 does not spill). Other shapes, with 64-bit indices: 4x4x16 26.0 / 4.64,
+// 4x8x8 27.8 / 4.65, 2x8x16 27.0 / 4.86, 8x8x8 29.0 / 5.06, 4x8x16 27.1 / 5.00, 8x4x16 27.3 /
+// 5.12, 8x2x16 28.3 / 4.90, 4x4x8 (two waves) 31.5 / 4.84 ms.
 //
 // The boxes alternate, so one barrier per field is enough: the box written for field i was last
 // read for field i - 2, and a wave passes the barrier of field i - 1 only after those reads.
@@ -81,17 +84,17 @@ struct GroupSrc : BoxStencil<GroupGeo<ORD, KO>, Coef<ORD>> {
   double* slots;        // this lane's parked values, NT apart
   const double* F;
   long P;
-  int off[G::PER];      // grid offsets of this lane's staged cells
+  unsigned off[G::PER]; // byte offsets of this lane's staged cells in a field
   int cel[G::PER];      // box indices of this lane's staged cells
   double pf[G::PER];    // the next field's cells, in flight
-  long gc;              // flat index of the lane's point (clamped into the grid)
+  unsigned gc;          // byte offset of the lane's point (clamped into the grid) in a field
   static constexpr int kParkSlots = G::SLOTS;
 
   __device__ __forceinline__ GroupSrc(double* mem, const double* F_, const Scales& sc_,
                                       const Dims& d, int ox, int oy, int oz, int t)
       : Box(mem, sc_), boxes(mem), slots(mem + 2 * G::VOL + t), F(F_), P(d.P) {
     c = (G::lx(t) + G::H) * G::SX + (G::ly(t) + G::H) * G::SY + (G::lz(t) + G::H);
-    gc = lane_point<G>(d, ox, oy, oz, t);
+    gc = (unsigned)lane_point<G>(d, ox, oy, oz, t) << 3;
     const int o[3] = {ox, oy, oz};
 #pragma unroll
     for (int k = 0; k < G::PER; ++k) {
@@ -101,7 +104,7 @@ struct GroupSrc : BoxStencil<GroupGeo<ORD, KO>, Coef<ORD>> {
       int g[3];
 #pragma unroll
       for (int a = 0; a < 3; ++a) g[a] = map_axis<MODE>(o[a] + cc[a] - G::H, d.S[a], d.ng);
-      off[k] = (g[0] * d.S[1] + g[1]) * d.S[2] + g[2];
+      off[k] = (unsigned)((g[0] * d.S[1] + g[1]) * d.S[2] + g[2]) << 3;
     }
     fetch(RhsOrder::at(0));
   }
@@ -115,7 +118,7 @@ struct GroupSrc : BoxStencil<GroupGeo<ORD, KO>, Coef<ORD>> {
     const int n = cells(f);
 #pragma unroll
     for (int k = 0; k < G::PER; ++k)
-      if (k < n) pf[k] = u[off[k]];
+      if (k < n) pf[k] = *at_byte(u, off[k]);
     __builtin_amdgcn_sched_barrier(0);   // keep the loads here, ahead of the work they overlap
   }
 
@@ -129,7 +132,7 @@ struct GroupSrc : BoxStencil<GroupGeo<ORD, KO>, Coef<ORD>> {
     if (at + 1 < RhsOrder::N) fetch(RhsOrder::at(at + 1));
   }
 
-  __device__ __forceinline__ double center(int f) const { return F[(long)f * P + gc]; }
+  __device__ __forceinline__ double center(int f) const { return *at_byte(F + (long)f * P, gc); }
   __device__ __forceinline__ void park(int i, double x) { slots[i * G::NT] = x; }
   __device__ __forceinline__ double parked(int i) const { return slots[i * G::NT]; }
 };

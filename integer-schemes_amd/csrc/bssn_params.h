@@ -10,6 +10,8 @@
 
 #include <stddef.h>
 
+#include <type_traits>
+
 #define BSSN_NF 24
 #define BSSN_ND 138
 #define BSSN_MAXTAP 9
@@ -168,6 +170,14 @@ __device__ __forceinline__ Scales scales_from_pack(const double* S, int ord, dou
     w.sko[a] = uniform(w.sko[a]);
   }
   return w;
+}
+
+// The element of a field (uniform base) at a 32-bit byte offset: the base stays in scalar
+// registers and the offset is one vector register, without 64-bit address arithmetic per access.
+template <class T>
+__device__ __forceinline__ T* at_byte(T* field, unsigned offset) {
+  using C = std::conditional_t<std::is_const_v<T>, const char, char>;
+  return reinterpret_cast<T*>(reinterpret_cast<C*>(field) + offset);
 }
 
 // Keep a value where it is computed: an empty volatile asm that claims to rewrite x. The

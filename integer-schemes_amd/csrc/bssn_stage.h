@@ -88,8 +88,11 @@ constexpr int fused_depth() {
 // cannot hold them longer; else BSSN_WB_LEAD phases ahead.
 template <int KIND, bool NEAR = false>
 struct StageOut {
+  // the lane's point: its byte offset in a field (NEAR, fields below 4 GiB) or its index
+  using Point = std::conditional_t<NEAR, unsigned, long>;
   const StageArgs& A;
-  long P, gp;
+  long P;
+  Point gp;
   bool valid;
   double gnew[6], anew[6];
 
@@ -103,7 +106,7 @@ struct StageOut {
   double pu[NU ? BSSN_NF : 1], pk[NK ? BSSN_NF : 1], pp[NF ? BSSN_NF : 1];
   bool deferred;
 
-  __device__ __forceinline__ StageOut(const StageArgs& a, long P_, long gp_, bool v,
+  __device__ __forceinline__ StageOut(const StageArgs& a, long P_, Point gp_, bool v,
                                       bool defer = false)
       : A(a), P(P_), gp(gp_), valid(v), deferred(defer) {
 #pragma unroll
@@ -111,11 +114,19 @@ struct StageOut {
       if (!defer) load(f);
   }
 
+  // field f of a state at the lane's point
+  template <class T>
+  __device__ __forceinline__ T& at(T* state, int f) const {
+    if constexpr (NEAR)
+      return *at_byte(state + (long)f * P, gp);
+    else
+      return state[(long)f * P + gp];
+  }
+
   __device__ __forceinline__ void load(int f) {
-    const long i = (long)f * P + gp;
-    if constexpr (NU) pu[f] = A.U[i];
-    if constexpr (NK) pk[f] = A.K1[i];
-    if constexpr (NF) pp[f] = A.FP[i];
+    if constexpr (NU) pu[f] = at(A.U, f);
+    if constexpr (NK) pk[f] = at(A.K1, f);
+    if constexpr (NF) pp[f] = at(A.FP, f);
   }
 
   // the bssn_rhs_point phase that stores field f, and the one that loads its operands
@@ -147,30 +158,29 @@ struct StageOut {
     } else {
       if (f == CHI) u = u < A.chi_floor ? A.chi_floor : u;
       if (f == ALPHA) u = u < A.alpha_floor ? A.alpha_floor : u;
-      A.Uout[(long)f * P + gp] = u;
+      at(A.Uout, f) = u;
     }
   }
 
   __device__ __forceinline__ void put(int f, double k) {
     if (!valid) return;
-    const long i = (long)f * P + gp;
     if constexpr (KIND == KIND_RHS) {
-      A.Y[i] = k;
+      at(A.Y, f) = k;
     } else if constexpr (KIND == KIND_RK1) {            // y + (dt/2) k1 ; S = k1
-      A.Y[i] = pu[f] + A.c0 * k;
-      A.K1[i] = k;
+      at(A.Y, f) = pu[f] + A.c0 * k;
+      at(A.K1, f) = k;
     } else if constexpr (KIND == KIND_RK2) {            // y + c0 k ; S = S + 2 k  (RK2, RK3)
-      A.Y[i] = pu[f] + A.c0 * k;
-      A.K1[i] = pk[f] + 2.0 * k;
+      at(A.Y, f) = pu[f] + A.c0 * k;
+      at(A.K1, f) = pk[f] + 2.0 * k;
     } else if constexpr (KIND == KIND_RK4) {            // y + (dt/6) (S + k4)
       final_value(f, pu[f] + A.c0 * (pk[f] + k));
     } else if constexpr (KIND == KIND_MS1) {            // y + dt (a20 k0 + a21 k1) ; store k1
-      A.Y[i] = pu[f] + A.dt * (A.c0 * pp[f] + A.c1 * k);
-      A.K1[i] = k;
+      at(A.Y, f) = pu[f] + A.dt * (A.c0 * pp[f] + A.c1 * k);
+      at(A.K1, f) = k;
     } else if constexpr (KIND == KIND_MS2) {            // y + dt (a30 k0 + a31 k1 + a32 k2)
       const double k0 = pp[f], k1 = pk[f];
-      A.Y[i] = pu[f] + A.dt * (A.c0 * k0 + A.c1 * k1 + A.c2 * k);
-      A.FP[i] = MS_B0 * k0 + MS_B1 * k1 + MS_B2 * k;
+      at(A.Y, f) = pu[f] + A.dt * (A.c0 * k0 + A.c1 * k1 + A.c2 * k);
+      at(A.FP, f) = MS_B0 * k0 + MS_B1 * k1 + MS_B2 * k;
     } else {                                            // MS3: y + dt (b0 k0 + ... + b3 k3)
       static_assert(KIND == KIND_MS3, "unknown stage kind");
       final_value(f, pu[f] + A.dt * (pp[f] + MS_B3 * k));
@@ -184,8 +194,8 @@ struct StageOut {
       enforce_point(gnew, anew);
 #pragma unroll
       for (int q = 0; q < 6; ++q) {
-        A.Uout[(long)(GT0 + q) * P + gp] = gnew[q];
-        A.Uout[(long)(AT0 + q) * P + gp] = anew[q];
+        at(A.Uout, GT0 + q) = gnew[q];
+        at(A.Uout, AT0 + q) = anew[q];
       }
     }
   }
