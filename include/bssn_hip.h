@@ -288,8 +288,9 @@ int bssn_batch_create(bssn_batch** out, void* plan, size_t plan_bytes, int nblk,
                       long long pool_doubles, void* stream);
 void bssn_batch_destroy(bssn_batch* b);
 
-/* Launch shape of the batched stage kernels: 0 = one workgroup per brick (default); N > 0
- * (a multiple of 8) = N persistent waves pulling bricks from per-XCD queues. */
+/* Launch shape of the batched stage kernels: 0 = one workgroup per brick (default; a brick is a
+ * wave's own or, for batches of enough and full enough blocks, shared by four waves); N > 0
+ * (a multiple of 8) = N persistent waves pulling wave-private bricks from per-XCD queues. */
 int bssn_batch_set_launch(bssn_batch* b, int persistent_waves);
 
 /* Interior (interior = 1) or padded point count of the batch; -1 for a null handle. */

@@ -648,6 +648,9 @@ struct bssn_batch {
   BlockDesc* blk = nullptr;          // device block table
   BrickList full{}, inner{}, ghost{};
   int grid_full = 0, grid_inner = 0, grid_ghost = 0;   // one workgroup per brick
+  BrickList sfull{}, sinner{};       // the same points in bricks shared by four waves
+  int grid_sfull = 0, grid_sinner = 0;
+  bool shared_full = false, shared_inner = false;   // which of the two a launch takes
   int* ctr = nullptr;                // device queue counters
   int persistent = 0;                // 0, or the persistent wave count
   const long long* i8pre = nullptr;  // device: 5 prefix arrays of the INT8 bundle passes
@@ -663,48 +666,46 @@ size_t align_up(size_t n) { return (n + kAlign - 1) & ~(kAlign - 1); }
 
 int cdiv(int n, int e) { return (n + e - 1) / e; }
 
-// Brick lists of one batch, built on the host. A brick of the padded block holds a ghost point
-// unless it lies inside [ng, S - ng) on every axis.
-struct HostLists {
-  std::vector<BrickItem> full, inner, ghost;
-  int cb_full[BATCH_CHUNKS + 1], cb_inner[BATCH_CHUNKS + 1], cb_ghost[BATCH_CHUNKS + 1];
-};
+// Brick lists of one batch, built on the host: padded blocks, interiors and ghost bricks in
+// wave-private bricks, and padded blocks and interiors in bricks shared by four waves.
+enum ListKind { L_FULL, L_INNER, L_GHOST, L_SFULL, L_SINNER, L_COUNT };
 
-void block_bricks(int b, const int* S, int ng, std::vector<BrickItem>* full,
-                  std::vector<BrickItem>* inner, std::vector<BrickItem>* ghost) {
-  auto pack = [](int x, int y, int z) { return x | (y << 10) | (z << 20); };
-  const int E[3] = {BSSN_BRICK_X, BSSN_BRICK_Y, BSSN_BRICK_Z};
-  for (int x = 0; x < S[0]; x += E[0])
-    for (int y = 0; y < S[1]; y += E[1])
-      for (int z = 0; z < S[2]; z += E[2]) {
-        if (full) full->push_back({b, pack(x, y, z)});
-        if (ghost) {
+struct Brick {
+  int e[3];
+};
+constexpr Brick kWaveBrick = {{BSSN_BRICK_X, BSSN_BRICK_Y, BSSN_BRICK_Z}};
+constexpr Brick kSharedBrick = {{BSSN_GROUP_X, BSSN_GROUP_Y, BSSN_GROUP_Z}};
+
+// The bricks of list `kind` of block b (S padded extents): a brick of the padded block is a ghost
+// brick unless it lies inside [ng, S - ng) on every axis.
+template <class Fn>
+void block_bricks(ListKind kind, const int* S, int ng, Fn&& add) {
+  const Brick& B = kind == L_SFULL || kind == L_SINNER ? kSharedBrick : kWaveBrick;
+  const int lo = kind == L_INNER || kind == L_SINNER ? ng : 0;
+  for (int x = lo; x < S[0] - lo; x += B.e[0])
+    for (int y = lo; y < S[1] - lo; y += B.e[1])
+      for (int z = lo; z < S[2] - lo; z += B.e[2]) {
+        if (kind == L_GHOST) {
           const int o[3] = {x, y, z};
           bool inside = true;
           for (int a = 0; a < 3; ++a)
-            inside = inside && o[a] >= ng && o[a] + E[a] <= S[a] - ng;
-          if (!inside) ghost->push_back({b, pack(x, y, z)});
+            inside = inside && o[a] >= ng && o[a] + B.e[a] <= S[a] - ng;
+          if (inside) continue;
         }
+        add(x | (y << 10) | (z << 20));
       }
-  if (inner)
-    for (int x = ng; x < S[0] - ng; x += E[0])
-      for (int y = ng; y < S[1] - ng; y += E[1])
-        for (int z = ng; z < S[2] - ng; z += E[2]) inner->push_back({b, pack(x, y, z)});
 }
 
-long list_count(int nblk, const int* S, int ng, int which) {
+long list_count(int nblk, const int* S, int ng, ListKind kind) {
   long n = 0;
   for (int b = 0; b < nblk; ++b) {
     const int* s = S + 3 * b;
-    if (which == 0) {
-      n += (long)cdiv(s[0], BSSN_BRICK_X) * cdiv(s[1], BSSN_BRICK_Y) * cdiv(s[2], BSSN_BRICK_Z);
-    } else if (which == 1) {
-      n += (long)cdiv(s[0] - 2 * ng, BSSN_BRICK_X) * cdiv(s[1] - 2 * ng, BSSN_BRICK_Y) *
-           cdiv(s[2] - 2 * ng, BSSN_BRICK_Z);
+    if (kind == L_GHOST) {
+      block_bricks(kind, s, ng, [&](int) { ++n; });
     } else {
-      std::vector<BrickItem> g;
-      block_bricks(b, s, ng, nullptr, nullptr, &g);
-      n += (long)g.size();
+      const Brick& B = kind == L_SFULL || kind == L_SINNER ? kSharedBrick : kWaveBrick;
+      const int g2 = kind == L_INNER || kind == L_SINNER ? 2 * ng : 0;
+      n += (long)cdiv(s[0] - g2, B.e[0]) * cdiv(s[1] - g2, B.e[1]) * cdiv(s[2] - g2, B.e[2]);
     }
   }
   return n;
@@ -735,6 +736,20 @@ std::vector<BrickItem> chunked(const std::vector<std::vector<BrickItem>>& per_bl
     cb[c + 1] = (int)out.size();
   }
   return out;
+}
+
+// Whether a launch over `points` takes the shared bricks: more wave-private bricks than the chip
+// holds at once (one per SIMD, 4 x 256; below that a launch is one brick's latency long, and the
+// wave-private one's is the shorter), fields below 4 GiB (32-bit byte offsets), and enough of the
+// shared bricks' lanes with a point (a block extent of 8 or 24 along z leaves half a brick
+// empty). FD4, blocks of 16 x 16 x n: RK4 step (interiors) at n = 8 / 12 / 16 / 20 / 24 / 32,
+// fill 0.5 / 0.75 / 1 / 0.63 / 0.75 / 1: wave-private 1.83 / 2.63 / 3.51 / 2.81 / 3.26 / 3.20,
+// shared 1.91 / 2.22 / 2.60 / 2.50 / 2.65 / 2.25 ms; RHS (padded) of 16 x 16 x 12 / 16 x 16 x 16
+// blocks, fill 0.47 / 0.58: 1.03 / 1.24 against 1.16 / 1.17 ms.
+constexpr double kSharedFill = 0.55;
+bool take_shared(long wave_bricks, long shared_bricks, long long points, long long largest) {
+  const double lanes = (double)(BSSN_GROUP_X * BSSN_GROUP_Y * BSSN_GROUP_Z) * shared_bricks;
+  return wave_bricks > 4 * 256 && largest < (1LL << 29) && (double)points >= kSharedFill * lanes;
 }
 
 int flat_grid(const int* cb) {
@@ -787,9 +802,10 @@ BatchArgs batch_args(const bssn_batch* b, bool interior, const double* S16, doub
                      double sigma) {
   BatchArgs a{};
   a.blk = b->blk;
-  a.list = interior ? b->inner : b->full;
-  a.ctr = b->ctr;
   a.persistent = b->persistent;
+  a.shared = !b->persistent && (interior ? b->shared_inner : b->shared_full);
+  a.list = a.shared ? (interior ? b->sinner : b->sfull) : (interior ? b->inner : b->full);
+  a.ctr = b->ctr;
   a.interior = interior ? 1 : 0;
   a.base = make_scal(S16, dt, t);
   a.cahd_c = S16[1];
@@ -801,6 +817,7 @@ BatchArgs batch_args(const bssn_batch* b, bool interior, const double* S16, doub
 int run_batch(const bssn_batch* b, const StageArgs& s, const BatchArgs& a, int ord, bool ko,
               int mode, hipStream_t st) {
   int grid = a.interior ? b->grid_inner : b->grid_full;
+  if (a.shared) grid = a.interior ? b->grid_sinner : b->grid_sfull;
   if (b->persistent) {
     TRY(check_hip(launch_batch_reset(b->ctr, st), "batch queue reset"));
     grid = b->persistent;
@@ -818,7 +835,8 @@ size_t bssn_batch_plan_bytes(int nblk, const int* S, int ng) {
   for (int b = 0; b < 3 * nblk; ++b)
     if (S[b] - 2 * ng < 1) return 0;
   size_t n = align_up(sizeof(BlockDesc) * (size_t)nblk);
-  for (int w = 0; w < 3; ++w) n += align_up(sizeof(BrickItem) * (size_t)list_count(nblk, S, ng, w));
+  for (int k = 0; k < L_COUNT; ++k)
+    n += align_up(sizeof(BrickItem) * (size_t)list_count(nblk, S, ng, (ListKind)k));
   n += align_up(sizeof(long long) * 5 * ((size_t)nblk + 1));   // INT8 bundle pass prefixes
   return n + align_up(sizeof(int) * BATCH_CHUNKS);
 }
@@ -833,9 +851,10 @@ int bssn_batch_create(bssn_batch** out, void* plan, size_t plan_bytes, int nblk,
   if (plan_bytes < need)
     return fail(BSSN_E_ARG, "plan buffer too small: need " + std::to_string(need) + " bytes");
   std::vector<BlockDesc> desc((size_t)nblk);
-  std::vector<std::vector<BrickItem>> pf((size_t)nblk), pi((size_t)nblk), pg((size_t)nblk);
+  std::vector<std::vector<BrickItem>> per[L_COUNT];
+  for (auto& p : per) p.resize((size_t)nblk);
   std::vector<long long> pre(5 * ((size_t)nblk + 1), 0);
-  long long interior = 0, padded = 0, doff = 0;
+  long long interior = 0, padded = 0, doff = 0, largest = 0;
   for (int b = 0; b < nblk; ++b) {
     const int* s = S + 3 * b;
     BlockDesc& d = desc[(size_t)b];
@@ -850,16 +869,18 @@ int bssn_batch_create(bssn_batch** out, void* plan, size_t plan_bytes, int nblk,
       d.S[a] = s[a];
       d.h[a] = h[3 * b + a];
     }
-    block_bricks(b, s, ng, &pf[(size_t)b], &pi[(size_t)b], &pg[(size_t)b]);
+    for (int k = 0; k < L_COUNT; ++k)
+      block_bricks((ListKind)k, s, ng,
+                   [&](int org) { per[k][(size_t)b].push_back({b, org}); });
+    largest = std::max(largest, (long long)s[0] * s[1] * s[2]);
     interior += (long long)(s[0] - 2 * ng) * (s[1] - 2 * ng) * (s[2] - 2 * ng);
     padded += (long long)s[0] * s[1] * s[2];
   }
-  HostLists L;
-  L.full = chunked(pf, L.cb_full);
-  L.inner = chunked(pi, L.cb_inner);
-  L.ghost = chunked(pg, L.cb_ghost);
+  std::vector<BrickItem> list[L_COUNT];
+  int cb[L_COUNT][BATCH_CHUNKS + 1];
+  for (int k = 0; k < L_COUNT; ++k) list[k] = chunked(per[k], cb[k]);
 
-  // plan image: block table | full | interior | ghost bricks | counters
+  // plan image: block table | brick lists | INT8 prefixes | counters
   std::vector<unsigned char> img(need, 0);
   size_t pos = 0;
   auto put = [&](const void* src, size_t bytes) {
@@ -869,9 +890,9 @@ int bssn_batch_create(bssn_batch** out, void* plan, size_t plan_bytes, int nblk,
     return at;
   };
   const size_t o_blk = put(desc.data(), sizeof(BlockDesc) * desc.size());
-  const size_t o_full = put(L.full.data(), sizeof(BrickItem) * L.full.size());
-  const size_t o_inner = put(L.inner.data(), sizeof(BrickItem) * L.inner.size());
-  const size_t o_ghost = put(L.ghost.data(), sizeof(BrickItem) * L.ghost.size());
+  size_t o_list[L_COUNT];
+  for (int k = 0; k < L_COUNT; ++k)
+    o_list[k] = put(list[k].data(), sizeof(BrickItem) * list[k].size());
   const size_t o_pre = put(pre.data(), sizeof(long long) * pre.size());
   const size_t o_ctr = pos;
   hipStream_t st = (hipStream_t)stream;
@@ -886,17 +907,18 @@ int bssn_batch_create(bssn_batch** out, void* plan, size_t plan_bytes, int nblk,
   bt->interior_pts = interior;
   bt->padded_pts = padded;
   bt->blk = (BlockDesc*)(base + o_blk);
-  bt->full.items = (const BrickItem*)(base + o_full);
-  bt->inner.items = (const BrickItem*)(base + o_inner);
-  bt->ghost.items = (const BrickItem*)(base + o_ghost);
-  for (int c = 0; c <= BATCH_CHUNKS; ++c) {
-    bt->full.cb[c] = L.cb_full[c];
-    bt->inner.cb[c] = L.cb_inner[c];
-    bt->ghost.cb[c] = L.cb_ghost[c];
+  BrickList* to[L_COUNT] = {&bt->full, &bt->inner, &bt->ghost, &bt->sfull, &bt->sinner};
+  int* grid[L_COUNT] = {&bt->grid_full, &bt->grid_inner, &bt->grid_ghost, &bt->grid_sfull,
+                        &bt->grid_sinner};
+  for (int k = 0; k < L_COUNT; ++k) {
+    to[k]->items = (const BrickItem*)(base + o_list[k]);
+    for (int i = 0; i <= BATCH_CHUNKS; ++i) to[k]->cb[i] = cb[k][i];
+    *grid[k] = flat_grid(cb[k]);
   }
-  bt->grid_full = flat_grid(L.cb_full);
-  bt->grid_inner = flat_grid(L.cb_inner);
-  bt->grid_ghost = flat_grid(L.cb_ghost);
+  bt->shared_full = take_shared((long)list[L_FULL].size(), (long)list[L_SFULL].size(), padded,
+                                largest);
+  bt->shared_inner = take_shared((long)list[L_INNER].size(), (long)list[L_SINNER].size(),
+                                 interior, largest);
   bt->ctr = (int*)(base + o_ctr);
   bt->i8pre = (const long long*)(base + o_pre);
   for (int k = 0; k < 5; ++k) bt->i8tot[k] = pre[(size_t)k * (nblk + 1) + nblk];

@@ -21,6 +21,7 @@
 
 #include "bssn_algebra.h"
 #include "bssn_brick.h"
+#include "bssn_group.h"
 #include "bssn_hip.h"
 #include "bssn_kernels.h"
 #include "bssn_params.h"
@@ -56,6 +57,49 @@ __device__ __forceinline__ int next_item(const BatchArgs& b, int* chunk, int* ro
   return -1;
 }
 
+// A block of the batch as one launch's grid: extents, per-block scales and scalars (formed on the
+// device in the host's rounding) and the stage's buffers at the block's offset. What is the same
+// for the whole brick is moved to scalar registers: the block table is read by vector loads, and
+// as vector values the six buffer pointers and the extents would live through the whole kernel.
+template <int ORD>
+struct BatchBlock {
+  Dims d;
+  Scales w;
+  Scal sc;
+  StageArgs a;
+  long off;             // pool offset of the block
+
+  __device__ __forceinline__ BatchBlock(const StageArgs& args, const BatchArgs& b,
+                                        const BlockDesc& blk) {
+    d.ng = uniform(blk.ng);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      d.S[a] = uniform(blk.S[a]);
+      d.lo[a] = b.interior ? d.ng : 0;
+      d.n[a] = b.interior ? d.S[a] - 2 * d.ng : d.S[a];
+    }
+    d.P = (long)d.S[0] * d.S[1] * d.S[2];
+    off = uniform(blk.off);
+    w = make_scales(blk.h, ORD, b.sigma);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      w.s1[a] = uniform(w.s1[a]);
+      w.s2[a] = uniform(w.s2[a]);
+      w.sm[a] = uniform(w.sm[a]);
+      w.sko[a] = uniform(w.sko[a]);
+    }
+    sc = with_ssl(b.base, args.tdev, args.toff);
+    sc.cahd = uniform(cahd_factor(b.cahd_c, blk.h[0], b.dt));
+    a = args;
+    a.Yin = shifted(args.Yin, off);
+    a.U = shifted(args.U, off);
+    a.Y = shifted(args.Y, off);
+    a.K1 = shifted(args.K1, off);
+    a.FP = shifted(args.FP, off);
+    a.Uout = shifted(args.Uout, off);
+  }
+};
+
 // one brick of one block, by the single-grid wave program
 template <int ORD, bool KO, int MODE, int KIND>
 __device__ __forceinline__ void batch_brick(double* lds, const StageArgs& args,
@@ -63,42 +107,18 @@ __device__ __forceinline__ void batch_brick(double* lds, const StageArgs& args,
   using G = Geo<ORD, KO>;
   const BrickItem item = b.list.items[it];
   const BlockDesc blk = b.blk[item.blk];
-  Dims d;
-  d.ng = blk.ng;
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    d.S[a] = blk.S[a];
-    d.lo[a] = b.interior ? blk.ng : 0;
-    d.n[a] = b.interior ? blk.S[a] - 2 * blk.ng : blk.S[a];
-  }
-  d.P = (long)blk.S[0] * blk.S[1] * blk.S[2];
-  const int ox = item.org & 1023, oy = (item.org >> 10) & 1023, oz = (item.org >> 20) & 1023;
-  Scales w = make_scales(blk.h, ORD, b.sigma);
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    w.s1[a] = uniform(w.s1[a]);
-    w.s2[a] = uniform(w.s2[a]);
-    w.sm[a] = uniform(w.sm[a]);
-    w.sko[a] = uniform(w.sko[a]);
-  }
-  Scal sc = with_ssl(b.base, args.tdev, args.toff);
-  sc.cahd = uniform(cahd_factor(b.cahd_c, blk.h[0], b.dt));
-  StageArgs a = args;
-  a.Yin = shifted(args.Yin, blk.off);
-  a.U = shifted(args.U, blk.off);
-  a.Y = shifted(args.Y, blk.off);
-  a.K1 = shifted(args.K1, blk.off);
-  a.FP = shifted(args.FP, blk.off);
-  a.Uout = shifted(args.Uout, blk.off);
+  const BatchBlock<ORD> B(args, b, blk);
+  const int org = uniform(item.org);
+  const int ox = org & 1023, oy = (org >> 10) & 1023, oz = (org >> 20) & 1023;
   using Src = WaveSrc<ORD, KO, MODE, RhsOrder, fused_depth<KIND, ORD>()>;
   if constexpr (MODE == LINK) {
-    Src src(lds, args.Yin, blk.off, b.link + 2 * blk.moff, b.pool_n, w, d, ox, oy, oz, lane);
-    StageOut<KIND> out(a, d.P, src.gc, lane_valid<G>(d, ox, oy, oz, lane), true);
-    bssn_rhs_point<KO>(src, sc, out);
+    Src src(lds, args.Yin, B.off, b.link + 2 * blk.moff, b.pool_n, B.w, B.d, ox, oy, oz, lane);
+    StageOut<KIND> out(B.a, B.d.P, src.gc, lane_valid<G>(B.d, ox, oy, oz, lane), true);
+    bssn_rhs_point<KO>(src, B.sc, out);
   } else {
-    Src src(lds, a.Yin, w, d, ox, oy, oz, lane);
-    StageOut<KIND> out(a, d.P, src.gc, lane_valid<G>(d, ox, oy, oz, lane), true);
-    bssn_rhs_point<KO>(src, sc, out);
+    Src src(lds, B.a.Yin, B.w, B.d, ox, oy, oz, lane);
+    StageOut<KIND> out(B.a, B.d.P, src.gc, lane_valid<G>(B.d, ox, oy, oz, lane), true);
+    bssn_rhs_point<KO>(src, B.sc, out);
   }
 }
 
@@ -123,11 +143,44 @@ void k_fused_batch(StageArgs args, BatchArgs b) {
   }
 }
 
+// The same on bricks shared by four waves (bssn_group.h), one workgroup per brick of the list;
+// equal results.
+template <int ORD, bool KO, int MODE, int KIND>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(2, 2)))
+void k_fused_batch_group(StageArgs args, BatchArgs b) {
+  using G = GroupGeo<ORD, KO>;
+  static_assert(G::NT == 256, "launch bounds");
+  __shared__ double mem[G::LDS_DOUBLES];
+  int chunk = 0, round = 0;
+  const int it = next_item(b, &chunk, &round);   // b.persistent is 0: the same for every lane
+  if (it < 0) return;
+  const BrickItem item = b.list.items[it];
+  const BlockDesc blk = b.blk[item.blk];
+  const BatchBlock<ORD> B(args, b, blk);
+  const int org = uniform(item.org);
+  const int ox = org & 1023, oy = (org >> 10) & 1023, oz = (org >> 20) & 1023;
+  const int t = (int)threadIdx.x;
+  using Src = GroupSrc<ORD, KO, MODE>;
+  if constexpr (MODE == LINK) {
+    Src src(mem, args.Yin, B.off, b.link + 2 * blk.moff, b.pool_n, B.w, B.d, ox, oy, oz, t);
+    StageOut<KIND, true> out(B.a, B.d.P, src.gc, lane_valid<G>(B.d, ox, oy, oz, t), true);
+    bssn_rhs_point<KO>(src, B.sc, out);
+  } else {
+    Src src(mem, B.a.Yin, B.w, B.d, ox, oy, oz, t);
+    StageOut<KIND, true> out(B.a, B.d.P, src.gc, lane_valid<G>(B.d, ox, oy, oz, t), true);
+    bssn_rhs_point<KO>(src, B.sc, out);
+  }
+}
+
 template <int ORD, bool KO, int MODE, int KIND>
 static hipError_t launch_batch_t(const StageArgs& a, const BatchArgs& b, int grid,
                                  hipStream_t st) {
   using G = Geo<ORD, KO>;
-  if (b.persistent)
+  if (b.shared)
+    hipLaunchKernelGGL((k_fused_batch_group<ORD, KO, MODE, KIND>), dim3(grid), dim3(256), 0, st,
+                       a, b);
+  else if (b.persistent)
     hipLaunchKernelGGL((k_fused_batch<ORD, KO, MODE, true, KIND>), dim3(grid), dim3(G::NT), 0,
                        st, a, b);
   else

@@ -38,7 +38,7 @@ struct GroupGeo {
   static constexpr int R = Coef<ORD>::R;                  // FD reach
   static constexpr int RK = KO ? Coef<ORD>::RK : 0;       // KO reach
   static constexpr int H = R > RK ? R : RK;               // box halo
-  static constexpr int BX = 4, BY = 4, BZ = 16;           // brick
+  static constexpr int BX = BSSN_GROUP_X, BY = BSSN_GROUP_Y, BZ = BSSN_GROUP_Z;  // brick
   static constexpr int NT = BX * BY * BZ;                 // lanes (four waves)
   static constexpr int NX = BX + 2 * H, NY = BY + 2 * H, NZ = BZ + 2 * H;   // box extents
   // dense rows and planes: the 16 lanes of one LDS access phase read one z row of the brick, 16
@@ -82,9 +82,11 @@ struct GroupSrc : BoxStencil<GroupGeo<ORD, KO>, Coef<ORD>> {
   using Box::lds;
   double* boxes;        // two boxes
   double* slots;        // this lane's parked values, NT apart
-  const double* F;
+  const double* F;      // stencil source state (LINK: the pool)
+  const double* Fc;     // the block's state (centre values)
   long P;
-  unsigned off[G::PER]; // byte offsets of this lane's staged cells in a field
+  unsigned off[G::PER]; // byte offsets of this lane's staged cells in a field (LINK: pool offsets)
+  int psrc[MODE == LINK ? G::PER : 1];   // LINK: field stride of each staged cell's block
   int cel[G::PER];      // box indices of this lane's staged cells
   double pf[G::PER];    // the next field's cells, in flight
   unsigned gc;          // byte offset of the lane's point (clamped into the grid) in a field
@@ -92,9 +94,9 @@ struct GroupSrc : BoxStencil<GroupGeo<ORD, KO>, Coef<ORD>> {
 
   __device__ __forceinline__ GroupSrc(double* mem, const double* F_, const Scales& sc_,
                                       const Dims& d, int ox, int oy, int oz, int t)
-      : Box(mem, sc_), boxes(mem), slots(mem + 2 * G::VOL + t), F(F_), P(d.P) {
-    c = (G::lx(t) + G::H) * G::SX + (G::ly(t) + G::H) * G::SY + (G::lz(t) + G::H);
-    gc = (unsigned)lane_point<G>(d, ox, oy, oz, t) << 3;
+      : Box(mem, sc_), boxes(mem), slots(mem + 2 * G::VOL + t), F(F_), Fc(F_), P(d.P) {
+    static_assert(MODE != LINK, "LINK sources take the pool and the link map");
+    place(d, ox, oy, oz, t);
     const int o[3] = {ox, oy, oz};
 #pragma unroll
     for (int k = 0; k < G::PER; ++k) {
@@ -109,6 +111,48 @@ struct GroupSrc : BoxStencil<GroupGeo<ORD, KO>, Coef<ORD>> {
     fetch(RhsOrder::at(0));
   }
 
+  // LINK: a block of a batch, as WaveSrc's (ng >= H; pool below 2^29 doubles), but the box of
+  // this larger brick may reach past the padded block where the brick passes the interior's end:
+  // such cells, which no lane with a point reads, are clamped into the block.
+  __device__ __forceinline__ GroupSrc(double* mem, const double* pool, long boff,
+                                      const int* lmap, long long pool_n, const Scales& sc_,
+                                      const Dims& d, int ox, int oy, int oz, int t)
+      : Box(mem, sc_), boxes(mem), slots(mem + 2 * G::VOL + t), F(pool), Fc(pool + boff),
+        P(d.P) {
+    static_assert(MODE == LINK, "the link constructor is for LINK sources");
+    place(d, ox, oy, oz, t);
+    const int o[3] = {ox, oy, oz};
+#pragma unroll
+    for (int k = 0; k < G::PER; ++k) {
+      const int e = kCells<G>.c[t + k * G::NT];
+      const int cc[3] = {e & 31, (e >> 5) & 31, (e >> 10) & 31};
+      cel[k] = cc[0] * G::SX + cc[1] * G::SY + cc[2];
+      int g[3];
+      bool inner = true;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        g[a] = map_axis<CLAMP>(o[a] + cc[a] - G::H, d.S[a], d.ng);
+        inner = inner && g[a] >= d.ng && g[a] < d.S[a] - d.ng;
+      }
+      const int q = (g[0] * d.S[1] + g[1]) * d.S[2] + g[2];
+      off[k] = (unsigned)((int)boff + q);
+      psrc[k] = (int)d.P;
+      if (!inner) {
+        const int2 m = reinterpret_cast<const int2*>(lmap)[q];
+        if (link_entry_ok(m.x, m.y, pool_n)) {
+          off[k] = (unsigned)m.x;
+          psrc[k] = m.y;
+        }
+      }
+    }
+    fetch(RhsOrder::at(0));
+  }
+
+  __device__ __forceinline__ void place(const Dims& d, int ox, int oy, int oz, int t) {
+    c = (G::lx(t) + G::H) * G::SX + (G::ly(t) + G::H) * G::SY + (G::lz(t) + G::H);
+    gc = (unsigned)lane_point<G>(d, ox, oy, oz, t) << 3;
+  }
+
   __device__ __forceinline__ static int cells(int f) {
     return needs_edges(f) ? G::PER : G::PER_FACES;
   }
@@ -118,7 +162,12 @@ struct GroupSrc : BoxStencil<GroupGeo<ORD, KO>, Coef<ORD>> {
     const int n = cells(f);
 #pragma unroll
     for (int k = 0; k < G::PER; ++k)
-      if (k < n) pf[k] = *at_byte(u, off[k]);
+      if (k < n) {
+        if constexpr (MODE == LINK)
+          pf[k] = *at_byte(F, (off[k] + (unsigned)(f * psrc[k])) << 3);
+        else
+          pf[k] = *at_byte(u, off[k]);
+      }
     __builtin_amdgcn_sched_barrier(0);   // keep the loads here, ahead of the work they overlap
   }
 
@@ -132,7 +181,7 @@ struct GroupSrc : BoxStencil<GroupGeo<ORD, KO>, Coef<ORD>> {
     if (at + 1 < RhsOrder::N) fetch(RhsOrder::at(at + 1));
   }
 
-  __device__ __forceinline__ double center(int f) const { return *at_byte(F + (long)f * P, gc); }
+  __device__ __forceinline__ double center(int f) const { return *at_byte(Fc + (long)f * P, gc); }
   __device__ __forceinline__ void park(int i, double x) { slots[i * G::NT] = x; }
   __device__ __forceinline__ double parked(int i) const { return slots[i * G::NT]; }
 };

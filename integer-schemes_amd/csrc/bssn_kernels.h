@@ -117,6 +117,7 @@ struct BatchArgs {
   BrickList list;
   int* ctr;          // BATCH_CHUNKS queue counters (zeroed before each persistent launch)
   int persistent;    // 0: one workgroup per brick; else waves pull bricks from the queues
+  int shared;        // the list holds bricks shared by four waves (one workgroup per brick)
   int interior;      // the list covers block interiors (else whole padded blocks)
   Scal base;         // shared scalars; cahd is set per block from its spacing
   double cahd_c, dt, sigma;

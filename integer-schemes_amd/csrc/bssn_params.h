@@ -29,6 +29,11 @@
 #endif
 static_assert(BSSN_BRICK_X * BSSN_BRICK_Y * BSSN_BRICK_Z == 64, "a brick is one 64-lane wave");
 
+// Brick shared by the four waves of a workgroup (bssn_group.h); host brick lists use it too.
+#define BSSN_GROUP_X 4
+#define BSSN_GROUP_Y 4
+#define BSSN_GROUP_Z 16
+
 namespace bssn {
 
 // Halo handling of the stencil source (see bssn_brick.h).
@@ -128,6 +133,13 @@ __device__ __forceinline__ double uniform(double x) {
   const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)u);
   const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(u >> 32));
   return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ long uniform(long x) {
+  const int lo = __builtin_amdgcn_readfirstlane((int)x);
+  const int hi = __builtin_amdgcn_readfirstlane((int)(x >> 32));
+  return ((long)hi << 32) | (unsigned)lo;
 }
 
 // The SSL factor exp(-t^2 / (2 sig^2)), formed on the device at the evaluation time: sc.ssl_t,

@@ -49,6 +49,10 @@ def waves(shape, seed, periodic=False, ng=0):
     return F
 
 
+def waves_of(n, ng, seed):
+    return waves([v + 2 * ng for v in n], seed, True, ng)
+
+
 def bricks(shape):
     return int(np.prod([(n + 3) // 4 for n in shape]))
 
@@ -94,21 +98,29 @@ def test_steps(interior, order, integrator, bc):
     assert err.max() < TOL, err
 
 
-@pytest.mark.parametrize("n", [(42, 39, 50), (34, 61, 64)])
-def test_equals_batched_form(n):
-    """One block through the batched kernels: the same bits."""
-    print(f"[case] batch {n}", flush=True)
-    batch = BlockBatch([Block(n=n, h=H3)], ng=3, device=DEV)
+@pytest.mark.parametrize("sizes,order", [([(42, 39, 50)], 4), ([(34, 61, 64)], 6),
+                                         ([(16, 17, 15), (12, 20, 33), (9, 16, 16)] * 8, 4),
+                                         ([(20, 8, 31), (33, 12, 48)] * 4, 8)])
+@pytest.mark.parametrize("waves", [0, 64])
+def test_batched_form_equals_single_grid(sizes, order, waves):
+    """Blocks through the batched kernels (shared bricks; persistent waves: wave-private bricks)
+    and one by one through the single-grid ones: the same bits."""
+    print(f"[case] batch {sizes[:3]} order {order} waves {waves}", flush=True)
+    ng = 3 if order == 4 else 4
+    h = [tuple(v * (1 + 0.1 * (b % 3)) for v in H3) for b in range(len(sizes))]
+    batch = BlockBatch([Block(n=n, h=q) for n, q in zip(sizes, h)], ng=ng, device=DEV)
+    assert sum(bricks(n) for n in sizes) > 1024
+    batch.set_launch(waves)
     U = batch.empty_pool()
-    batch.view(U, 0).copy_(torch.from_numpy(waves([v + 6 for v in n], 7, True, 3)))
-    F = batch.view(U, 0).clone()
-    out, one = torch.empty_like(U), torch.empty_like(F)
-    batch.rhs_into(U, out, P, 0.02, order=4, ko_sigma=0.1)
-    S16 = scalars(P, *H3, 0.02, 0.0)
-    S16[3] = H3[0]
-    rhs_into(F, one, S16, 4, 0.1)
-    assert torch.equal(batch.view(out, 0), one)
-    evo = BSSNEvolution(Grid(*n, *H3, ng=3), P, order=4, ko_sigma=0.1)
-    evo.step_(F, 0.0, 0.02)
-    batch.step_(U, 0.0, 0.02, P, order=4, ko_sigma=0.1, bc="periodic")
-    assert torch.equal(batch.view(U, 0), F)
+    for b, n in enumerate(sizes):
+        batch.view(U, b).copy_(torch.from_numpy(waves_of(n, ng, b)))
+    start, out = U.clone(), torch.empty_like(U)
+    batch.rhs_into(U, out, P, 0.02, order=order, ko_sigma=0.1)
+    batch.step_(U, 0.0, 0.02, P, order=order, ko_sigma=0.1, bc="periodic")
+    for b, (n, q) in enumerate(zip(sizes, h)):
+        F = batch.view(start, b).clone()
+        one = torch.empty_like(F)
+        rhs_into(F, one, scalars(P, *q, 0.02, 0.0), order, 0.1)
+        assert torch.equal(batch.view(out, b), one), b
+        BSSNEvolution(Grid(*n, *q, ng=ng), P, order=order, ko_sigma=0.1).step_(F, 0.0, 0.02)
+        assert torch.equal(batch.view(U, b), F), b
