@@ -352,8 +352,8 @@ struct WaveSrc : BoxStencil<Geo<ORD, KO>, Coef<ORD>> {
 
   // LINK: a block of a batch (pool offset boff, link map lmap of its padded points). Cells in
   // the block's interior are read in place; a ghost cell is read where the map points, or in
-  // place if the entry would reach outside the pool (pool_n doubles). Needs ng >= H (the box
-  // stays inside the padded block) and a pool below 2^29 doubles.
+  // place if the entry would reach outside the pool (pool_n doubles). Needs ng >= H and a pool
+  // below 2^29 doubles.
   __device__ __forceinline__ WaveSrc(double* lds_, const double* pool, long boff,
                                      const int* lmap, long long pool_n, const Scales& sc_,
                                      const Dims& d, int ox, int oy, int oz, int lane)
@@ -372,7 +372,9 @@ struct WaveSrc : BoxStencil<Geo<ORD, KO>, Coef<ORD>> {
       bool inner = true;
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
-        g[a] = o[a] + cc[a] - G::H;
+        // clamped: the box of a brick that passes the interior's end may leave the padded block
+        // (no lane with a point reads those cells, but the map has no entry for them)
+        g[a] = map_axis<CLAMP>(o[a] + cc[a] - G::H, d.S[a], d.ng);
         inner = inner && g[a] >= d.ng && g[a] < d.S[a] - d.ng;
       }
       const int q = (g[0] * d.S[1] + g[1]) * d.S[2] + g[2];

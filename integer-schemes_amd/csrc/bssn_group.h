@@ -111,9 +111,7 @@ struct GroupSrc : BoxStencil<GroupGeo<ORD, KO>, Coef<ORD>> {
     fetch(RhsOrder::at(0));
   }
 
-  // LINK: a block of a batch, as WaveSrc's (ng >= H; pool below 2^29 doubles), but the box of
-  // this larger brick may reach past the padded block where the brick passes the interior's end:
-  // such cells, which no lane with a point reads, are clamped into the block.
+  // LINK: a block of a batch, as WaveSrc's (ng >= H; pool below 2^29 doubles).
   __device__ __forceinline__ GroupSrc(double* mem, const double* pool, long boff,
                                       const int* lmap, long long pool_n, const Scales& sc_,
                                       const Dims& d, int ox, int oy, int oz, int t)
