@@ -126,6 +126,57 @@ __device__ __forceinline__ void raise_A(const double* A, const double* ig, doubl
   *AA = contract_sym(Aup, A);
 }
 
+// Christoffels and the metric part of the conformal Ricci tensor: from d_k gt_q and gt^ij,
+// C2 = Gamma^m_ij, CalGt = gt^ij Gamma^m_ij, and Rt (holding -1/2 gt^kl d_k d_l gt_ij) completed.
+__device__ __forceinline__ void ricci_metric(const double (&dg)[3][6], const double* ig,
+                                             double (&C2)[3][6], double* CalGt, double* Rt) {
+  double C1[3][6];   // Gamma_k(ij), first index lowered
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+#pragma unroll
+    for (int q = 0; q < 6; ++q) {
+      const int i = pi_(q), j = pj_(q);
+      C1[k][q] = 0.5 * (dg[j][sym(k, i)] + dg[i][sym(k, j)] - dg[k][q]);
+    }
+#pragma unroll
+  for (int m = 0; m < 3; ++m)
+#pragma unroll
+    for (int q = 0; q < 6; ++q)
+      C2[m][q] = ig[sym(m, 0)] * C1[0][q] + ig[sym(m, 1)] * C1[1][q] + ig[sym(m, 2)] * C1[2][q];
+#pragma unroll
+  for (int m = 0; m < 3; ++m) CalGt[m] = contract_sym(ig, C2[m]);
+  //   Rt_ij += CalGt^k (Gamma_ijk + Gamma_jik)/2
+  //          + gt^lm (Gamma^k_li Gamma_jkm + Gamma^k_lj Gamma_ikm + Gamma^k_im Gamma_klj)
+  // with the raised forms Gu[i][k][m] = gt^ml Gamma^k_li and gt^ml Gamma_klj.
+  double Gu[3][3][3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+      for (int m = 0; m < 3; ++m)
+        Gu[i][k][m] = ig[sym(m, 0)] * C2[k][sym(0, i)] + ig[sym(m, 1)] * C2[k][sym(1, i)] +
+                      ig[sym(m, 2)] * C2[k][sym(2, i)];
+#pragma unroll
+  for (int q = 0; q < 6; ++q) {
+    const int i = pi_(q), j = pj_(q);
+    double t = 0.0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) t += CalGt[k] * (C1[i][sym(j, k)] + C1[j][sym(i, k)]);
+    double u = 0.0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+      for (int m = 0; m < 3; ++m) {
+        const double gd = ig[sym(m, 0)] * C1[k][sym(0, j)] + ig[sym(m, 1)] * C1[k][sym(1, j)] +
+                          ig[sym(m, 2)] * C1[k][sym(2, j)];
+        u += Gu[i][k][m] * C1[j][sym(k, m)] + Gu[j][k][m] * C1[i][sym(k, m)] +
+             C2[k][sym(i, m)] * gd;
+      }
+    Rt[q] += 0.5 * t + u;
+  }
+}
+
 template <bool KO, class Src, class Out>
 __device__ __forceinline__ void bssn_rhs_point(Src& s, const Scal& P, Out& o) {
   // Values formed early and used late: the gt rates without their Lie terms (gt phase to At
@@ -197,51 +248,7 @@ __device__ __forceinline__ void bssn_rhs_point(Src& s, const Scal& P, Out& o) {
 #pragma unroll
       for (int i = 0; i < 3; ++i) keep(P_ADV + i, b[i]);
     }
-    double C1[3][6];   // Gamma_k(ij), first index lowered
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-#pragma unroll
-      for (int q = 0; q < 6; ++q) {
-        const int i = pi_(q), j = pj_(q);
-        C1[k][q] = 0.5 * (dg[j][sym(k, i)] + dg[i][sym(k, j)] - dg[k][q]);
-      }
-#pragma unroll
-    for (int m = 0; m < 3; ++m)
-#pragma unroll
-      for (int q = 0; q < 6; ++q)
-        C2[m][q] = ig[sym(m, 0)] * C1[0][q] + ig[sym(m, 1)] * C1[1][q] + ig[sym(m, 2)] * C1[2][q];
-#pragma unroll
-    for (int m = 0; m < 3; ++m) CalGt[m] = contract_sym(ig, C2[m]);
-    //   Rt_ij += CalGt^k (Gamma_ijk + Gamma_jik)/2
-    //          + gt^lm (Gamma^k_li Gamma_jkm + Gamma^k_lj Gamma_ikm + Gamma^k_im Gamma_klj)
-    // with the raised forms Gu[i][k][m] = gt^ml Gamma^k_li and gt^ml Gamma_klj.
-    double Gu[3][3][3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int k = 0; k < 3; ++k)
-#pragma unroll
-        for (int m = 0; m < 3; ++m)
-          Gu[i][k][m] = ig[sym(m, 0)] * C2[k][sym(0, i)] + ig[sym(m, 1)] * C2[k][sym(1, i)] +
-                        ig[sym(m, 2)] * C2[k][sym(2, i)];
-#pragma unroll
-    for (int q = 0; q < 6; ++q) {
-      const int i = pi_(q), j = pj_(q);
-      double t = 0.0;
-#pragma unroll
-      for (int k = 0; k < 3; ++k) t += CalGt[k] * (C1[i][sym(j, k)] + C1[j][sym(i, k)]);
-      double u = 0.0;
-#pragma unroll
-      for (int k = 0; k < 3; ++k)
-#pragma unroll
-        for (int m = 0; m < 3; ++m) {
-          const double gd = ig[sym(m, 0)] * C1[k][sym(0, j)] + ig[sym(m, 1)] * C1[k][sym(1, j)] +
-                            ig[sym(m, 2)] * C1[k][sym(2, j)];
-          u += Gu[i][k][m] * C1[j][sym(k, m)] + Gu[j][k][m] * C1[i][sym(k, m)] +
-               C2[k][sym(i, m)] * gd;
-        }
-      Rt[q] += 0.5 * t + u;
-    }
+    ricci_metric(dg, ig, C2, CalGt, Rt);
   }
 #pragma unroll
   for (int q = 0; q < 6; ++q) {
@@ -511,17 +518,7 @@ __device__ __forceinline__ void bssn_constraints_point(Src& s, Out& o) {
   double g[6], ig[6];
 #pragma unroll
   for (int q = 0; q < 6; ++q) g[q] = s.center(GT0 + q);
-  {
-    const double a00 = g[3] * g[5] - g[4] * g[4];
-    const double a01 = g[2] * g[4] - g[1] * g[5];
-    const double a02 = g[1] * g[4] - g[2] * g[3];
-    const double a11 = g[0] * g[5] - g[2] * g[2];
-    const double a12 = g[1] * g[2] - g[0] * g[4];
-    const double a22 = g[0] * g[3] - g[1] * g[1];
-    const double idet = 1.0 / (g[0] * a00 + g[1] * a01 + g[2] * a02);
-    ig[0] = a00 * idet; ig[1] = a01 * idet; ig[2] = a02 * idet;
-    ig[3] = a11 * idet; ig[4] = a12 * idet; ig[5] = a22 * idet;
-  }
+  inverse_sym(g, ig);
   double dg[3][6], Rt[6];
 #pragma unroll
   for (int q = 0; q < 6; ++q) {
@@ -532,41 +529,19 @@ __device__ __forceinline__ void bssn_constraints_point(Src& s, Out& o) {
                     2.0 * (ig[1] * s.d2(0, 1) + ig[2] * s.d2(0, 2) + ig[4] * s.d2(1, 2)));
   }
   double C2[3][6], CalGt[3];
-  {
-    double C1[3][6];
+  // the metric, which the Ricci tensor does not use, waits in the source's slots if it has any
+  constexpr bool PARK = ParkSlots<Src>::value > 0;
+  if constexpr (PARK) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
-#pragma unroll
-      for (int q = 0; q < 6; ++q) {
-        const int i = pi_(q), j = pj_(q);
-        C1[k][q] = 0.5 * (dg[j][sym(k, i)] + dg[i][sym(k, j)] - dg[k][q]);
-      }
-#pragma unroll
-    for (int m = 0; m < 3; ++m)
-#pragma unroll
-      for (int q = 0; q < 6; ++q)
-        C2[m][q] = ig[sym(m, 0)] * C1[0][q] + ig[sym(m, 1)] * C1[1][q] + ig[sym(m, 2)] * C1[2][q];
-#pragma unroll
-    for (int m = 0; m < 3; ++m) CalGt[m] = contract_sym(ig, C2[m]);
+    for (int q = 0; q < 6; ++q) s.park(q, g[q]);
+  }
+  ricci_metric(dg, ig, C2, CalGt, Rt);
+  if constexpr (PARK) {
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int q = 0; q < 6; ++q) {
-      const int i = pi_(q), j = pj_(q);
-      double t = 0.0, u = 0.0;
-#pragma unroll
-      for (int k = 0; k < 3; ++k) t += CalGt[k] * (C1[i][sym(j, k)] + C1[j][sym(i, k)]);
-#pragma unroll
-      for (int k = 0; k < 3; ++k)
-#pragma unroll
-        for (int m = 0; m < 3; ++m) {
-          const double gui = ig[sym(m, 0)] * C2[k][sym(0, i)] + ig[sym(m, 1)] * C2[k][sym(1, i)] +
-                             ig[sym(m, 2)] * C2[k][sym(2, i)];
-          const double guj = ig[sym(m, 0)] * C2[k][sym(0, j)] + ig[sym(m, 1)] * C2[k][sym(1, j)] +
-                             ig[sym(m, 2)] * C2[k][sym(2, j)];
-          const double gd = ig[sym(m, 0)] * C1[k][sym(0, j)] + ig[sym(m, 1)] * C1[k][sym(1, j)] +
-                            ig[sym(m, 2)] * C1[k][sym(2, j)];
-          u += gui * C1[j][sym(k, m)] + guj * C1[i][sym(k, m)] + C2[k][sym(i, m)] * gd;
-        }
-      Rt[q] += 0.5 * t + u;
+      BSSN_PIN(Rt[q]);
+      g[q] = s.parked(q);
     }
   }
   double chi, dchi[3];

@@ -13,11 +13,13 @@
 
 #include <math.h>
 
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
 #include "bssn_algebra.h"
 #include "bssn_brick.h"
+#include "bssn_group.h"
 #include "bssn_kernels.h"
 #include "bssn_params.h"
 
@@ -58,18 +60,25 @@ __device__ __forceinline__ double nanmax_d(double m, double v) {
   return (v > m || v != v) ? v : m;
 }
 
-template <int STORE>
-__device__ __forceinline__ void bundle_put(const BundleOut& o, int slot, long P, long gc,
+// array `slot` of the bundle at the lane's point: byte offset in a field (fields below 4 GiB) or
+// index
+template <int STORE, class Point>
+__device__ __forceinline__ void bundle_put(const BundleOut& o, int slot, long P, Point gc,
                                            double v, bool valid) {
+  constexpr bool WIDE = std::is_same_v<Point, long>;
   if constexpr (STORE == BS_F64) {
-    if (valid) o.D[(long)slot * P + gc] = v;
+    if (!valid) return;
+    if constexpr (WIDE)
+      o.D[(long)slot * P + gc] = v;
+    else
+      *at_byte(o.D + (long)slot * P, gc) = v;
   } else {
     if (!valid) return;
     // saturate to [-2^(k-1), 2^(k-1) - 1]; a NaN (which an integer mantissa cannot hold) stores
     // as the negative saturation value, like -inf, so the conversion below is always defined
     double m = rint(ldexp(v, o.e[slot]));
     m = !(m >= -o.lim) ? -o.lim : (m > o.lim - 1.0 ? o.lim - 1.0 : m);
-    const long i = (long)slot * P + gc;
+    const long i = (long)slot * P + (WIDE ? (long)gc : (long)(gc >> 3));
     if constexpr (STORE == BS_Q32) {
       ((int*)o.Q)[i] = (int)m;
     } else {
@@ -82,41 +91,40 @@ __device__ __forceinline__ void bundle_put(const BundleOut& o, int slot, long P,
   }
 }
 
-template <int ORD, int STORE>
-__global__ __launch_bounds__(64) void k_deriv_bundle(const double* __restrict__ F, BundleOut o,
-                                                     Dims d, Scales w) {
-  using G = Geo<ORD, false>;
-  __shared__ double lds[G::VOL];
+// Bricks shared by four waves, two boxes, a barrier per field (bssn_group.h), kFieldRun fields per
+// workgroup (blockIdx.y). What bounds the pass is the store of the 138 arrays (with the stencils
+// left out it takes as long): 4 x 4 x 16 bricks write rows of 128 B, where a wave's own 4 x 4 x 4
+// brick wrote pieces of 32 B, and the runs, dispatched one after the other, write 3 to 18 arrays
+// at a time instead of 138. 134^3, FD6 fp64 / 118^3, FD4 BFP32: 2.08 / 0.96 -> 1.33 / 0.50 ms (runs
+// of 1 / 3 / 4 / 8 / 24 fields: 1.38 / 1.35 / 1.37 / 1.43 / 1.48 and 0.53 / 0.50 / 0.51 / 0.51 /
+// 0.54). Rows that start on a 128 B line write a quarter faster (2.85 against 2.13 TB/s); the
+// caller's row pitch decides that.
+constexpr int kFieldRun = 2;
+static_assert(BSSN_NF % kFieldRun == 0, "whole runs");
+
+template <int ORD, int STORE, bool WIDE>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(ORD == 8 ? 2 : 4)))
+void k_deriv_bundle(const double* __restrict__ F, BundleOut o, Dims d, Scales w) {
+  using G = GroupGeo<ORD, false>;
+  __shared__ double mem[2 * G::VOL];
   int ox, oy, oz;
   if (!brick_origin<G>(d, &ox, &oy, &oz)) return;
-  const int lane = (int)threadIdx.x;
-  const bool valid = lane_valid<G>(d, ox, oy, oz, lane);
-  // FD4 fp64 / BFP32 stores: two fields in flight, stepped in pairs so each staging slot is a
-  // constant (256^3: two-pass RHS with KO 28.6 -> 26.8 ms, BFP32 with fixed exponents 15.9 ->
-  // 13.1 ms). The BFP48 store and FD order 6 keep one (their extra registers cost more waves
-  // per SIMD than the second field gains: BFP48 19.0 -> 21.1 ms with two).
-  constexpr int DEPTH = ORD == 4 && STORE != BS_Q48 ? 2 : 1;
-  WaveSrc<ORD, false, CLAMP, StateOrder, DEPTH> s(lds, F, w, d, ox, oy, oz, lane);
-  auto field = [&](int f, auto slot) {
-    s.template stage_slot<decltype(slot)::value>(f);
-    double v[9];
+  const int t = (int)threadIdx.x, f0 = (int)blockIdx.y * kFieldRun;
+  const bool valid = lane_valid<G>(d, ox, oy, oz, t);
+  GroupSrc<ORD, false, CLAMP, StateOrder, WIDE> s(mem, F, w, d, ox, oy, oz, t, f0);
+#pragma unroll 1
+  for (int i = 0; i < kFieldRun; ++i) {
+    const int f = f0 + i, sl = s2slot(f);
+    s.stage_in(f, i & 1, i + 1 < kFieldRun ? f + 1 : -1);
 #pragma unroll
-    for (int a = 0; a < 3; ++a) v[a] = s.d1(a);
-    const int sl = s2slot(f);
-    if (sl >= 0) {
-#pragma unroll
-      for (int q = 0; q < 6; ++q) v[3 + q] = s.d2(pi_(q), pj_(q));
-    }
-#pragma unroll
-    for (int a = 0; a < 3; ++a) bundle_put<STORE>(o, 3 * f + a, d.P, s.gc, v[a], valid);
+    for (int a = 0; a < 3; ++a) bundle_put<STORE>(o, 3 * f + a, d.P, s.gc, s.d1(a), valid);
     if (sl >= 0) {
 #pragma unroll
       for (int q = 0; q < 6; ++q)
-        bundle_put<STORE>(o, 72 + 6 * sl + q, d.P, s.gc, v[3 + q], valid);
+        bundle_put<STORE>(o, 72 + 6 * sl + q, d.P, s.gc, s.d2(pi_(q), pj_(q)), valid);
     }
-    __builtin_amdgcn_wave_barrier();
-  };
-  for_fields<DEPTH>(field);
+  }
 }
 
 template <int STORE>
@@ -124,8 +132,12 @@ static void launch_bundle_store(const double* F, const BundleOut& o, const Dims&
                                 const Scales& w, int ord, hipStream_t st) {
   with_order(ord, [&](auto oc) {
     constexpr int O = decltype(oc)::value;
-    hipLaunchKernelGGL((k_deriv_bundle<O, STORE>), dim3(brick_blocks<Geo<O, false>>(d)),
-                       dim3(64), 0, st, F, o, d, w);
+    using G = GroupGeo<O, false>;
+    const dim3 grid(brick_blocks<G>(d), BSSN_NF / kFieldRun);
+    if (d.P < kGroupPoints)
+      hipLaunchKernelGGL((k_deriv_bundle<O, STORE, false>), grid, dim3(G::NT), 0, st, F, o, d, w);
+    else
+      hipLaunchKernelGGL((k_deriv_bundle<O, STORE, true>), grid, dim3(G::NT), 0, st, F, o, d, w);
   });
 }
 
@@ -147,69 +159,80 @@ __global__ void k_put_scales(double* dst, BfpScales s) {
   if (i < BSSN_ND) dst[i] = s.inv[i];
 }
 
-// Per-array maxima with few atomics: each wave walks many bricks, keeps the running maxima in
-// registers (lane l holds arrays l, l + 64, l + 128) and ends with one atomicMax per array.
-template <int ORD>
-__global__ __launch_bounds__(64) void k_bundle_absmax(const double* __restrict__ F,
-                                                      unsigned long long* __restrict__ amax,
-                                                      Dims d, Scales w) {
-  using G = Geo<ORD, false>;
-  __shared__ double lds[G::VOL];
-  const int lane = (int)threadIdx.x;
+// Per-array maxima with few atomics: a workgroup takes one field (blockIdx.y) through many
+// bricks, a lane keeps the running maxima of the field's 3 or 9 arrays in registers, and the
+// workgroup ends with one atomicMax per array. With the fields inside the bricks every value needed a
+// reduction over the wave (138 of six steps per brick): that, not the stencils, was the time
+// (118^3, FD4: 1.23 -> 0.41 ms; 96 / 128 / 192 / 400 instead of 256 workgroups per field 0.46 /
+// 0.44 / 0.41 / 0.41).
+// EDGES: the 11 fields with second derivatives, else the 13 others.
+template <int ORD, bool EDGES, bool WIDE>
+__global__ __launch_bounds__(256) void k_bundle_absmax(const double* __restrict__ F,
+                                                       unsigned long long* __restrict__ amax,
+                                                       Dims d, Scales w) {
+  using G = GroupGeo<ORD, false>;
+  __shared__ double mem[2 * G::VOL];
+  constexpr int NA = EDGES ? 9 : 3;   // arrays of the field
+  const int t = (int)threadIdx.x, y = (int)blockIdx.y;
+  const int f = EDGES ? (y < KTR ? y : y + 1) : (y == 0 ? KTR : AT0 - 1 + y);
   const int nbx = (d.n[0] + G::BX - 1) / G::BX, nby = (d.n[1] + G::BY - 1) / G::BY,
             nbz = (d.n[2] + G::BZ - 1) / G::BZ;
   const int nb = nbx * nby * nbz;
-  double r0 = 0.0, r1 = 0.0, r2 = 0.0;
-  auto keep = [&](int slot, double v, bool valid) {
-    double a = valid ? fabs(v) : 0.0;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) a = nanmax_d(a, __shfl_xor(a, off, 64));
-    if (lane == (slot & 63)) {
-      const int q = slot >> 6;
-      if (q == 0) r0 = nanmax_d(r0, a);
-      else if (q == 1) r1 = nanmax_d(r1, a);
-      else r2 = nanmax_d(r2, a);
-    }
-  };
-  for (int L = (int)blockIdx.x; L < nb; L += (int)gridDim.x) {
-    const int bz = L % nbz, t = L / nbz, by = t % nby, bx = t / nby;
+  double m[NA] = {};
+  int box = 0;
+  for (int L = (int)blockIdx.x; L < nb; L += (int)gridDim.x, box ^= 1) {
+    const int bz = L % nbz, c = L / nbz, by = c % nby, bx = c / nby;
     const int ox = d.lo[0] + bx * G::BX, oy = d.lo[1] + by * G::BY, oz = d.lo[2] + bz * G::BZ;
-    const bool valid = lane_valid<G>(d, ox, oy, oz, lane);
-    // one field in flight (two measured no faster here)
-    WaveSrc<ORD, false, CLAMP, StateOrder> s(lds, F, w, d, ox, oy, oz, lane);
-    auto field = [&](int f, auto slot) {
-      s.template stage_slot<decltype(slot)::value>(f);
-      double v[9];
+    const bool valid = lane_valid<G>(d, ox, oy, oz, t);
+    GroupSrc<ORD, false, CLAMP, OneField<EDGES>, WIDE> s(mem, F + (long)f * d.P, w, d, ox, oy,
+                                                         oz, t);
+    s.stage_in(0, box, -1);   // the boxes alternate from brick to brick
 #pragma unroll
-      for (int a = 0; a < 3; ++a) v[a] = s.d1(a);
-      const int sl = s2slot(f);
-      if (sl >= 0) {
+    for (int a = 0; a < 3; ++a) m[a] = nanmax_d(m[a], valid ? fabs(s.d1(a)) : 0.0);
+    if constexpr (EDGES) {
 #pragma unroll
-        for (int q = 0; q < 6; ++q) v[3 + q] = s.d2(pi_(q), pj_(q));
-      }
-#pragma unroll
-      for (int a = 0; a < 3; ++a) keep(3 * f + a, v[a], valid);
-      if (sl >= 0) {
-#pragma unroll
-        for (int q = 0; q < 6; ++q) keep(72 + 6 * sl + q, v[3 + q], valid);
-      }
-      __builtin_amdgcn_wave_barrier();
-    };
-    for_fields<1>(field);
+      for (int q = 0; q < 6; ++q)
+        m[3 + q] = nanmax_d(m[3 + q], valid ? fabs(s.d2(pi_(q), pj_(q))) : 0.0);
+    }
   }
-  atomicMax(amax + lane, (unsigned long long)__double_as_longlong(r0));
-  atomicMax(amax + 64 + lane, (unsigned long long)__double_as_longlong(r1));
-  if (128 + lane < BSSN_ND)
-    atomicMax(amax + 128 + lane, (unsigned long long)__double_as_longlong(r2));
+  // one atomicMax per array and workgroup: the 138 maxima share nine cache lines, and at one per
+  // wave the atomics were most of the pass
+  __shared__ double wave_max[4][NA];
+#pragma unroll
+  for (int i = 0; i < NA; ++i) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) m[i] = nanmax_d(m[i], __shfl_xor(m[i], off, 64));
+    if ((t & 63) == 0) wave_max[t >> 6][i] = m[i];
+  }
+  __syncthreads();
+  if (t < NA) {
+    double a = wave_max[0][t];
+#pragma unroll
+    for (int v = 1; v < 4; ++v) a = nanmax_d(a, wave_max[v][t]);
+    atomicMax(amax + (t < 3 ? 3 * f + t : 72 + 6 * s2slot(f) + t - 3),
+              (unsigned long long)__double_as_longlong(a));
+  }
 }
 
 hipError_t launch_bundle_absmax(const double* F, unsigned long long* amax, const Dims& d,
                                 const Scales& w, int ord, hipStream_t st) {
   hipLaunchKernelGGL(k_clear_u64, dim3(1), dim3(256), 0, st, amax, BSSN_ND);
-  const unsigned grid = 2048;
   with_order(ord, [&](auto oc) {
     constexpr int O = decltype(oc)::value;
-    hipLaunchKernelGGL(k_bundle_absmax<O>, dim3(grid), dim3(64), 0, st, F, amax, d, w);
+    using G = GroupGeo<O, false>;
+    auto run = [&](auto edges, auto wide, int fields) {
+      const dim3 grid(std::min(256u, brick_blocks<G>(d)), fields);
+      hipLaunchKernelGGL((k_bundle_absmax<O, decltype(edges)::value, decltype(wide)::value>), grid,
+                         dim3(G::NT), 0, st, F, amax, d, w);
+    };
+    auto both = [&](auto wide) {
+      run(std::true_type(), wide, 11);
+      run(std::false_type(), wide, 13);
+    };
+    if (d.P < kGroupPoints)
+      both(std::false_type());
+    else
+      both(std::true_type());
   });
   return hipGetLastError();
 }
@@ -457,16 +480,19 @@ struct ConsOut {
   }
 };
 
-template <int ORD>
-__global__ __launch_bounds__(64) void k_constraints(const double* __restrict__ F,
-                                                    double* __restrict__ HM, Dims d, Scales w) {
-  using G = Geo<ORD, false>;
-  __shared__ double lds[G::VOL];
+// Bricks shared by four waves, two waves per SIMD (bssn_group.h). Like the fused kernels it waited
+// on memory at one wave per SIMD (376 registers): 150^3 FD4 0.80 -> 0.60 ms.
+template <int ORD, bool WIDE>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(2, 2)))
+void k_constraints(const double* __restrict__ F, double* __restrict__ HM, Dims d, Scales w) {
+  using G = GroupGeo<ORD, false>;
+  __shared__ double mem[2 * G::VOL + 6 * G::NT];   // two boxes and six parked values per lane
   int ox, oy, oz;
   if (!brick_origin<G>(d, &ox, &oy, &oz)) return;
-  const int lane = (int)threadIdx.x;
-  WaveSrc<ORD, false, CLAMP, ConsOrder> s(lds, F, w, d, ox, oy, oz, lane);
-  ConsOut o{HM, d.P, s.gc, lane_valid<G>(d, ox, oy, oz, lane)};
+  const int t = (int)threadIdx.x;
+  GroupSrc<ORD, false, CLAMP, ConsOrder, WIDE> s(mem, F, w, d, ox, oy, oz, t);
+  ConsOut o{HM, d.P, lane_point<G>(d, ox, oy, oz, t), lane_valid<G>(d, ox, oy, oz, t)};
   bssn_constraints_point(s, o);
 }
 
@@ -474,8 +500,13 @@ hipError_t launch_constraints(const double* F, double* HM, const Dims& d, const 
                               int ord, hipStream_t st) {
   with_order(ord, [&](auto oc) {
     constexpr int O = decltype(oc)::value;
-    hipLaunchKernelGGL(k_constraints<O>, dim3(brick_blocks<Geo<O, false>>(d)), dim3(64), 0, st,
-                       F, HM, d, w);
+    using G = GroupGeo<O, false>;
+    if (d.P < kGroupPoints)
+      hipLaunchKernelGGL((k_constraints<O, false>), dim3(brick_blocks<G>(d)), dim3(G::NT), 0, st,
+                         F, HM, d, w);
+    else
+      hipLaunchKernelGGL((k_constraints<O, true>), dim3(brick_blocks<G>(d)), dim3(G::NT), 0, st,
+                         F, HM, d, w);
   });
   return hipGetLastError();
 }

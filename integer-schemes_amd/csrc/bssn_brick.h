@@ -174,7 +174,8 @@ template <class G>
 __constant__ CellTable<G> kCells = CellTable<G>();
 
 // Field staging orders: the fused RHS stages in the order of bssn_rhs_point's phases; the
-// per-field loops (bundle, KO) in state order.
+// per-field loops (bundle, KO) in state order; edges(f): whether field f is staged with the edge
+// bars of its mixed derivatives.
 struct RhsOrder {
   // gt0..5 | chi | Gt0..2 | alpha | beta0..2 | At0..5 | K | B0..2
   static constexpr int N = BSSN_NF;
@@ -198,11 +199,13 @@ struct RhsOrder {
          : f == KTR ? 20
          : 21 + f - BB0;
   }
+  __host__ __device__ static constexpr bool edges(int f) { return needs_edges(f); }
 };
 struct StateOrder {
   static constexpr int N = BSSN_NF;
   __host__ __device__ static constexpr int at(int i) { return i; }
   __host__ __device__ static constexpr int pos(int f) { return f; }
+  __host__ __device__ static constexpr bool edges(int f) { return needs_edges(f); }
 };
 // the constraints: gt0..5 | chi | Gt0..2 | At0..5 | K (pos = N for the fields they do not use)
 struct ConsOrder {
@@ -219,6 +222,16 @@ struct ConsOrder {
          : f == KTR ? 16
          : N;
   }
+  __host__ __device__ static constexpr bool edges(int f) { return needs_edges(f); }
+};
+
+// one field by itself (field 0 of the source), with or without mixed derivatives
+template <bool EDGES>
+struct OneField {
+  static constexpr int N = 1;
+  __host__ __device__ static constexpr int at(int) { return 0; }
+  __host__ __device__ static constexpr int pos(int) { return 0; }
+  __host__ __device__ static constexpr bool edges(int) { return EDGES; }
 };
 
 // flat index of the lane's point, clamped into the grid (write-back index of invalid lanes)

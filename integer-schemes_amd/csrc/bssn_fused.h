@@ -71,7 +71,6 @@ void k_fused_group(StageArgs args, Dims d, Scales w, Scal sc) {
 // The shared form addresses a field by 32-bit byte offsets, so fields of 4 GiB and more (a state
 // of 103 GB: only the bare RHS fits the card) take the wave-private form too.
 constexpr unsigned kWaveBricks = 4 * 256;
-constexpr long kGroupPoints = 1L << 29;
 
 template <int ORD, bool KO, int MODE, int KIND, bool SDEV>
 static hipError_t launch_fused_t(const StageArgs& a, const Dims& d, const Scales& w,

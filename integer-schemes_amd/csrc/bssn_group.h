@@ -29,6 +29,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "bssn_brick.h"
 
 namespace bssn {
@@ -62,6 +64,9 @@ struct GroupGeo {
   static constexpr int LDS_DOUBLES = 2 * VOL + SLOTS * NT;
 };
 
+// Points of a field from which its bytes no longer fit 32-bit offsets (4 GiB).
+constexpr long kGroupPoints = 1L << 29;
+
 // Barrier of the workgroup that orders its LDS accesses (global loads and stores stay in
 // flight across it).
 __device__ __forceinline__ void group_barrier() {
@@ -73,8 +78,8 @@ __device__ __forceinline__ void group_barrier() {
 // Source of fields and derivatives for bssn_rhs_point over shared boxes: as WaveSrc with one
 // field in flight, with a workgroup barrier where WaveSrc relies on a wave's LDS order. Every
 // lane of the workgroup must run the whole stage sequence (lanes without a point of their own
-// stage cells for the others).
-template <int ORD, bool KO, int MODE>
+// stage cells for the others). WIDE: 64-bit addresses, for fields of 4 GiB and more.
+template <int ORD, bool KO, int MODE, class ORDER = RhsOrder, bool WIDE = false>
 struct GroupSrc : BoxStencil<GroupGeo<ORD, KO>, Coef<ORD>> {
   using G = GroupGeo<ORD, KO>;
   using Box = BoxStencil<G, Coef<ORD>>;
@@ -85,15 +90,18 @@ struct GroupSrc : BoxStencil<GroupGeo<ORD, KO>, Coef<ORD>> {
   const double* F;      // stencil source state (LINK: the pool)
   const double* Fc;     // the block's state (centre values)
   long P;
-  unsigned off[G::PER]; // byte offsets of this lane's staged cells in a field (LINK: pool offsets)
+  unsigned off[G::PER]; // byte offsets of this lane's staged cells in a field (LINK: pool
+                        // offsets in doubles, WIDE: offsets in doubles)
   int psrc[MODE == LINK ? G::PER : 1];   // LINK: field stride of each staged cell's block
   int cel[G::PER];      // box indices of this lane's staged cells
   double pf[G::PER];    // the next field's cells, in flight
-  unsigned gc;          // byte offset of the lane's point (clamped into the grid) in a field
+  std::conditional_t<WIDE, long, unsigned> gc;   // the lane's point, clamped into the grid: byte
+                                                 // offset in a field (WIDE: index)
   static constexpr int kParkSlots = G::SLOTS;
 
   __device__ __forceinline__ GroupSrc(double* mem, const double* F_, const Scales& sc_,
-                                      const Dims& d, int ox, int oy, int oz, int t)
+                                      const Dims& d, int ox, int oy, int oz, int t,
+                                      int first = ORDER::at(0))
       : Box(mem, sc_), boxes(mem), slots(mem + 2 * G::VOL + t), F(F_), Fc(F_), P(d.P) {
     static_assert(MODE != LINK, "LINK sources take the pool and the link map");
     place(d, ox, oy, oz, t);
@@ -106,9 +114,10 @@ struct GroupSrc : BoxStencil<GroupGeo<ORD, KO>, Coef<ORD>> {
       int g[3];
 #pragma unroll
       for (int a = 0; a < 3; ++a) g[a] = map_axis<MODE>(o[a] + cc[a] - G::H, d.S[a], d.ng);
-      off[k] = (unsigned)((g[0] * d.S[1] + g[1]) * d.S[2] + g[2]) << 3;
+      off[k] = (unsigned)((g[0] * d.S[1] + g[1]) * d.S[2] + g[2]);
+      if constexpr (!WIDE) off[k] <<= 3;
     }
-    fetch(RhsOrder::at(0));
+    fetch(first);
   }
 
   // LINK: a block of a batch, as WaveSrc's (ng >= H; pool below 2^29 doubles).
@@ -143,16 +152,17 @@ struct GroupSrc : BoxStencil<GroupGeo<ORD, KO>, Coef<ORD>> {
         }
       }
     }
-    fetch(RhsOrder::at(0));
+    fetch(ORDER::at(0));
   }
 
   __device__ __forceinline__ void place(const Dims& d, int ox, int oy, int oz, int t) {
     c = (G::lx(t) + G::H) * G::SX + (G::ly(t) + G::H) * G::SY + (G::lz(t) + G::H);
-    gc = (unsigned)lane_point<G>(d, ox, oy, oz, t) << 3;
+    gc = lane_point<G>(d, ox, oy, oz, t);
+    if constexpr (!WIDE) gc <<= 3;
   }
 
   __device__ __forceinline__ static int cells(int f) {
-    return needs_edges(f) ? G::PER : G::PER_FACES;
+    return ORDER::edges(f) ? G::PER : G::PER_FACES;
   }
 
   __device__ __forceinline__ void fetch(int f) {
@@ -163,23 +173,35 @@ struct GroupSrc : BoxStencil<GroupGeo<ORD, KO>, Coef<ORD>> {
       if (k < n) {
         if constexpr (MODE == LINK)
           pf[k] = *at_byte(F, (off[k] + (unsigned)(f * psrc[k])) << 3);
+        else if constexpr (WIDE)
+          pf[k] = u[off[k]];
         else
           pf[k] = *at_byte(u, off[k]);
       }
     __builtin_amdgcn_sched_barrier(0);   // keep the loads here, ahead of the work they overlap
   }
 
-  __device__ __forceinline__ void stage(int f) {
-    const int at = RhsOrder::pos(f), n = cells(f);
-    lds = boxes + (at & 1) * G::VOL;
+  // field f, loaded before, into a box; next: the field to load while f is used (-1: none)
+  __device__ __forceinline__ void stage_in(int f, int box, int next) {
+    const int n = cells(f);
+    lds = boxes + box * G::VOL;
 #pragma unroll
     for (int k = 0; k < G::PER; ++k)
       if (k < n) lds[cel[k]] = pf[k];
     group_barrier();
-    if (at + 1 < RhsOrder::N) fetch(RhsOrder::at(at + 1));
+    if (next >= 0) fetch(next);
+  }
+  __device__ __forceinline__ void stage(int f) {
+    const int at = ORDER::pos(f);
+    stage_in(f, at & 1, at + 1 < ORDER::N ? ORDER::at(at + 1) : -1);
   }
 
-  __device__ __forceinline__ double center(int f) const { return *at_byte(Fc + (long)f * P, gc); }
+  __device__ __forceinline__ double center(int f) const {
+    if constexpr (WIDE)
+      return Fc[(long)f * P + gc];
+    else
+      return *at_byte(Fc + (long)f * P, gc);
+  }
   __device__ __forceinline__ void park(int i, double x) { slots[i * G::NT] = x; }
   __device__ __forceinline__ double parked(int i) const { return slots[i * G::NT]; }
 };

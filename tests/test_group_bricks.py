@@ -17,10 +17,12 @@ import torch
 import oracle as O
 from conftest import gpu_available, normwise
 
+from bssn3d_hip import _lib
 from bssn3d_hip.batch import Block, BlockBatch
+from bssn3d_hip.constraints import ConstraintSolver
 from bssn3d_hip.evolve import BSSNEvolution
 from bssn3d_hip.grid import Grid
-from bssn3d_hip.rhs import rhs_into
+from bssn3d_hip.rhs import rhs_into, stream_handle
 from bssn3d_hip.state import PhysicsParams, scalars
 
 pytestmark = [pytest.mark.gpu,
@@ -124,3 +126,38 @@ def test_batched_form_equals_single_grid(sizes, order, waves):
         assert torch.equal(batch.view(out, b), one), b
         BSSNEvolution(Grid(*n, *q, ng=ng), P, order=order, ko_sigma=0.1).step_(F, 0.0, 0.02)
         assert torch.equal(batch.view(U, b), F), b
+
+
+@pytest.mark.parametrize("shape", [(5, 6, 7), (9, 4, 17), (20, 23, 31), (12, 13, 48)])
+@pytest.mark.parametrize("order", [4, 6, 8])
+def test_bundle_maxima_and_constraints(shape, order):
+    """The derivative bundle, its per-array maxima and the constraints. A derivative's rounding
+    error is bounded by eps times the number of roundings (under 64) times the sum of its
+    stencil's weights times max|u|; the maxima are those of the stored bundle exactly."""
+    print(f"[case] bundle {shape} order {order}", flush=True)
+    F = waves(shape, seed=order)
+    Fd = torch.from_numpy(F).to(DEV)
+    D = torch.empty((138,) + tuple(shape), dtype=torch.float64, device=DEV)
+    amax = torch.empty(138, dtype=torch.float64, device=DEV)
+    lib, st, h3 = _lib.load(), stream_handle(Fd.device), _lib.dbl(H3)
+    _lib.check(lib.bssn_deriv_bundle_f64(Fd.data_ptr(), D.data_ptr(), *shape, order, h3, st))
+    _lib.check(lib.bssn_deriv_bundle_absmax_f64(Fd.data_ptr(), amax.data_ptr(), *shape, order,
+                                                h3, st))
+    assert torch.equal(amax, D.abs().flatten(1).max(dim=1).values)
+    got, ref = D.cpu().numpy(), O.deriv_bundle(F, list(H3), order)
+    c1, c2 = (np.abs(O.stencil(k, order)).sum() for k in (0, 1))
+    for d in range(138):
+        if d < 72:
+            f, a = divmod(d, 3)
+            mag = c1 / H3[a]
+        else:
+            s, q = divmod(d - 72, 6)
+            f = O.IDX[O.S2_FIELDS[s]]
+            i, j = O.PAIRS[q]
+            mag = c2 / H3[i] ** 2 if i == j else c1 * c1 / (H3[i] * H3[j])
+        assert np.abs(got[d] - ref[d]).max() <= 64 * 2.2e-16 * mag * np.abs(F[f]).max(), d
+    grid = Grid(*[max(n - 2 * 2, 1) for n in shape], *H3, ng=(order // 2))
+    C = ConstraintSolver(grid, order=order).constraints(Fd)
+    err = normwise(torch.stack([C[k] for k in ("H", "M0", "M1", "M2")]).cpu().numpy(),
+                   O.constraints(F, list(H3), order))
+    assert err.max() < TOL, err
