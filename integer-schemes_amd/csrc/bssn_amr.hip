@@ -14,6 +14,8 @@
 // interior plus one ring, per (block, field), NaN-propagating like a max over an array.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "bssn_entries.h"
 #include "bssn_hip.h"
 #include "bssn_kernels.h"
@@ -253,7 +255,7 @@ hipError_t launch_prolong(double* pool, long long pool_n, const void* pts, long 
   return hipGetLastError();
 }
 
-// Separable whole-block prolongation: one workgroup per (job, field, x slab), a slab being
+// Separable whole-block prolongation: one workgroup per (job, field group, x slab), a slab being
 // PB_SLABS-th of the padded block's fine x planes. The x pass fills X[rx][ky][kz] (the slab's
 // fine x planes, coarse y and z window) from the parent, the y pass Y[rx][ry][kz] from X, and
 // the z sums are formed only at the points the job writes. Every fine x plane depends only on
@@ -261,34 +263,63 @@ hipError_t launch_prolong(double* pool, long long pool_n, const void* pts, long 
 // read clamped, so the taps of every sum are the clamped nodes of the per-point kernel, summed
 // in the same order. A job that is not a valid block of at most PB_WMAX padded nodes per axis
 // inside the pool (pool_n doubles) is skipped (the test is uniform across the workgroup, so no
-// thread reaches a barrier alone). Eight slabs of 256 threads (19.6 KB LDS, several workgroups
-// per CU): on the 384-block hierarchy (16^3 blocks) one fill takes 0.801 ms, against 0.801 /
-// 0.811 ms with 2 slabs of 512 / 4 of 256, and 0.883 ms with one 1024-thread workgroup per
-// (job, field) holding the whole block's passes (157 KB LDS, one workgroup per CU).
-#ifndef BSSN_PB_SLABS
-#define BSSN_PB_SLABS 8
-#endif
-#ifndef BSSN_PB_THREADS
-#define BSSN_PB_THREADS 256
-#endif
-constexpr int PB_SLABS = BSSN_PB_SLABS;
+// thread reaches a barrier alone). What bounds it is instruction issue, not its bytes: most of
+// it was turning indices into coordinates by integer division, for every field anew. A workgroup
+// now takes PB_FIELDS fields of a slab, a thread forms its columns, rows and points once, the next
+// field's coarse nodes are loaded while the current one's passes run, and a plane whose points
+// are all supplied but its ghost rows forms only those. 384-block hierarchy (16^3 blocks), the two
+// launches of a fill: 0.310 + 0.210 -> 0.144 + 0.102 ms (2 / 4 / 24 fields 0.189 + 0.129 / 0.153
+// + 0.106 / 0.167 + 0.097; 8 or 5 slabs 0.178 / 0.186 for the larger one at 4 fields; 384 / 512
+// threads 0.155 / 0.152).
+constexpr int PB_SLABS = 6;
+constexpr int PB_THREADS = 256;
+constexpr int PB_FIELDS = 8;
+static_assert(BSSN_NF % PB_FIELDS == 0, "field groups must tile the 24 fields");
 constexpr int PB_SW = (PB_WMAX + PB_SLABS - 1) / PB_SLABS;   // fine x planes per slab, at most
 
-__global__ __launch_bounds__(BSSN_PB_THREADS) void k_prolong_block(
+// Quotient of 0 <= i < 2^20 / PB_WMAX by a divisor known only at run time, 1 <= d <= PB_WMAX,
+// with a quotient below 2^11: m = 2^20 / d rounded up exceeds it by less than 1, so i m 2^-20
+// exceeds i / d by less than i 2^-20 < 1 / PB_WMAX and rounds down to the quotient. Two
+// instructions instead of about 40.
+struct SmallDiv {
+  unsigned m;
+  __device__ __forceinline__ explicit SmallDiv(int d) : m(((1u << 20) + d - 1) / d) {}
+  __device__ __forceinline__ int quot(int i) const { return (int)(((unsigned)i * m) >> 20); }
+};
+static_assert(PB_SW * PB_WMAX * PB_WMAX < (1 << 20) / PB_WMAX && PB_SW * PB_WMAX < (1 << 11),
+              "SmallDiv's range");
+
+// sum of the six taps at u[0], u[stride], ..., left to right from 0.0 (odd fine index), or the
+// coarse node itself (even)
+__device__ __forceinline__ double refine_1d(const double* u, int stride, bool odd) {
+#pragma clang fp contract(off)
+  double v = 0.0;
+#pragma unroll
+  for (int j = 0; j < 6; ++j) v = v + kWMid[j] * u[j * stride];
+  return odd ? v : u[2 * stride];
+}
+
+__global__ __launch_bounds__(PB_THREADS) void k_prolong_block(
     double* __restrict__ pool, const bssn_prolong_block* __restrict__ jobs, long long pool_n) {
 #pragma clang fp contract(off)
+  constexpr int NX = (PB_KMAX * PB_KMAX + PB_THREADS - 1) / PB_THREADS;
+  constexpr int NY = (PB_SW * PB_WMAX * PB_KMAX + PB_THREADS - 1) / PB_THREADS;
+  constexpr int NZ = (PB_SW * PB_WMAX * PB_WMAX + PB_THREADS - 1) / PB_THREADS;
+  constexpr int NV = 6 + (PB_SW + 1) / 2;         // coarse nodes under a slab's planes, at most
   __shared__ double X[PB_SW * PB_KMAX * PB_KMAX];
   __shared__ double Y[PB_SW * PB_WMAX * PB_KMAX];
   const int slab = (int)(blockIdx.x % PB_SLABS);
   const long jf = blockIdx.x / PB_SLABS;
-  const bssn_prolong_block jb = jobs[jf / BSSN_NF];
+  constexpr int NG = BSSN_NF / PB_FIELDS;
+  const bssn_prolong_block jb = jobs[jf / NG];
   if (!block_job_ok(jb, pool_n)) return;
-  const int f = (int)(jf % BSSN_NF);
+  const int f0 = (int)(jf % NG) * PB_FIELDS;
   const int W = jb.BS + 2 * jb.ng;
   const int sw = (W + PB_SLABS - 1) / PB_SLABS;
   const int x0 = slab * sw, nx = min(W, x0 + sw) - x0;
   if (nx <= 0) return;
-  const long sy = W, sx = (long)W * W, P = sx * W;
+  const int sy = W, sx = W * W;
+  const long P = (long)sx * W;
   int r0[3], kmin[3], K[3];
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
@@ -296,73 +327,132 @@ __global__ __launch_bounds__(BSSN_PB_THREADS) void k_prolong_block(
     kmin[a] = (r0[a] >> 1) - 2;
     K[a] = ((r0[a] + W - 1) >> 1) + 3 - kmin[a] + 1;
   }
-  const double* c = pool + jb.parent + (long)f * P;
-  const int nX = nx * K[1] * K[2];
-  for (int i = (int)threadIdx.x; i < nX; i += (int)blockDim.x) {
-    const int kz = i % K[2], ky = (i / K[2]) % K[1], xl = i / (K[2] * K[1]);
-    const int rx = r0[0] + x0 + xl;
-    const int ny = clampi(kmin[1] + ky, 0, W - 1), nz = clampi(kmin[2] + kz, 0, W - 1);
-    const double* row = c + (long)ny * sy + nz;
-    double v;
-    if ((rx & 1) == 0) {
-      v = row[(long)clampi(rx >> 1, 0, W - 1) * sx];
-    } else {
-      v = 0.0;
+  const int lo = jb.ng, hi = jb.ng + jb.BS, t = (int)threadIdx.x;
+  const SmallDiv dK2(K[2]), dW(W), dG(max(1, 2 * lo));
+
+  // What a thread does in the three passes is the same for every field: formed once.
+  // x pass: window columns (ky, kz), their offset in a parent plane and their place in X
+  int xsrc[NX], xdst[NX];
 #pragma unroll
-      for (int j = 0; j < 6; ++j) v = v + kWMid[j] * row[(long)clampi((rx >> 1) - 2 + j, 0, W - 1) * sx];
-    }
-    X[(xl * PB_KMAX + ky) * PB_KMAX + kz] = v;
+  for (int k = 0; k < NX; ++k) {
+    const int i = min(t + k * PB_THREADS, K[1] * K[2] - 1);
+    const int ky = dK2.quot(i), kz = i - ky * K[2];
+    xsrc[k] = clampi(kmin[1] + ky, 0, W - 1) * sy + clampi(kmin[2] + kz, 0, W - 1);
+    xdst[k] = ky * PB_KMAX + kz;
   }
-  __syncthreads();
-  const int nY = nx * W * K[2];
-  for (int i = (int)threadIdx.x; i < nY; i += (int)blockDim.x) {
-    const int kz = i % K[2], y = (i / K[2]) % W, xl = i / (K[2] * W);
-    const int ry = r0[1] + y;
-    const double* col = X + (long)xl * PB_KMAX * PB_KMAX + kz;
-    double v;
-    if ((ry & 1) == 0) {
-      v = col[((ry >> 1) - kmin[1]) * PB_KMAX];
+  // The y rows a plane needs: all of them, or, for a plane inside the block whose z face slabs
+  // come from neighbours, its 2 ng ghost rows only. Planes [0, a) and [a + ns, nx) of the slab are
+  // of the first kind, [a, a + ns) of the second.
+  const bool thin = lo > 0 && (jb.skip & (48 | 64)) == 48;
+  const int a = thin ? min(nx, max(0, lo - x0)) : nx;
+  const int ns = thin ? max(0, min(nx, hi - x0) - a) : 0;
+  const int full_rows = (nx - ns) * W, rows = full_rows + ns * 2 * lo;
+  auto row_at = [&](int r, int* xl, int* y) {
+    if (r < full_rows) {
+      const int p = dW.quot(r);
+      *y = r - p * W;
+      *xl = p < a ? p : p + ns;
     } else {
-      v = 0.0;
+      const int p = dG.quot(r - full_rows), q = r - full_rows - p * 2 * lo;
+      *y = q < lo ? q : q + jb.BS;
+      *xl = a + p;
+    }
+  };
+  // y pass: first tap in X | place in Y << 12 | odd << 24; -1: none
+  int yitem[NY];
 #pragma unroll
-      for (int j = 0; j < 6; ++j) v = v + kWMid[j] * col[((ry >> 1) - 2 + j - kmin[1]) * PB_KMAX];
+  for (int k = 0; k < NY; ++k) {
+    const int i = t + k * PB_THREADS, r = dK2.quot(i), kz = i - r * K[2];
+    yitem[k] = -1;
+    if (i < rows * K[2]) {
+      int xl, y;
+      row_at(r, &xl, &y);
+      const int ry = r0[1] + y;
+      yitem[k] = ((xl * PB_KMAX + (ry >> 1) - 2 - kmin[1]) * PB_KMAX + kz) |
+                 ((xl * PB_WMAX + y) * PB_KMAX + kz) << 12 | (ry & 1) << 24;
     }
-    Y[(xl * PB_WMAX + y) * PB_KMAX + kz] = v;
   }
-  __syncthreads();
-  const int lo = jb.ng, hi = jb.ng + jb.BS;
-  double* out = pool + jb.dst + (long)f * P;
-  for (int i = (int)threadIdx.x; i < nx * W * W; i += (int)blockDim.x) {
-    const int z = i % W, y = (i / W) % W, xl = i / (W * W), x = x0 + xl;
-    const bool ix = x >= lo && x < hi, iy = y >= lo && y < hi, iz = z >= lo && z < hi;
-    if (ix && iy && iz) {
-      if (!(jb.skip & 64)) continue;
-    } else {
-      // a face slab: ghost along exactly one axis, interior along the other two
-      if (iy && iz && (jb.skip & (x < lo ? 1 : 2))) continue;
-      if (ix && iz && (jb.skip & (y < lo ? 4 : 8))) continue;
-      if (ix && iy && (jb.skip & (z < lo ? 16 : 32))) continue;
-    }
-    const int rz = r0[2] + z;
-    const double* yy = Y + (xl * PB_WMAX + y) * PB_KMAX;
-    double v;
-    if ((rz & 1) == 0) {
-      v = yy[(rz >> 1) - kmin[2]];
-    } else {
-      v = 0.0;
+  // z pass: first tap in Y | point of the block << 12 | odd << 26; -1: not written
+  int zitem[NZ];
 #pragma unroll
-      for (int j = 0; j < 6; ++j) v = v + kWMid[j] * yy[(rz >> 1) - 2 + j - kmin[2]];
+  for (int k = 0; k < NZ; ++k) {
+    const int i = t + k * PB_THREADS, r = dW.quot(i), z = i - r * W;
+    zitem[k] = -1;
+    if (i < rows * W) {
+      int xl, y;
+      row_at(r, &xl, &y);
+      const int x = x0 + xl, rz = r0[2] + z;
+      const bool ix = x >= lo && x < hi, iy = y >= lo && y < hi, iz = z >= lo && z < hi;
+      // the interior only if asked for; a face slab (ghost along exactly one axis, interior along
+      // the other two) unless a neighbour supplies it
+      const bool skip = (ix && iy && iz) ? !(jb.skip & 64)
+                        : (iy && iz)     ? (jb.skip & (x < lo ? 1 : 2)) != 0
+                        : (ix && iz)     ? (jb.skip & (y < lo ? 4 : 8)) != 0
+                        : (ix && iy)     ? (jb.skip & (z < lo ? 16 : 32)) != 0
+                                         : false;
+      if (!skip)
+        zitem[k] = ((xl * PB_WMAX + y) * PB_KMAX + (rz >> 1) - 2 - kmin[2]) |
+                   ((x * W + y) * W + z) << 12 | (rz & 1) << 26;
     }
-    out[((long)x * W + y) * W + z] = v;
   }
+  const int k0 = ((r0[0] + x0) >> 1) - 2;
+  int plane[NV];                                   // offsets of the coarse planes
+#pragma unroll
+  for (int j = 0; j < NV; ++j) plane[j] = clampi(k0 + j, 0, W - 1) * sx;
+
+  auto run = [&](auto odd) {
+    constexpr int ODD = decltype(odd)::value;      // parity of the slab's first plane
+    double u[NX][NV];
+    auto load = [&](int f) {
+      const double* c = pool + jb.parent + (long)f * P;
+#pragma unroll
+      for (int k = 0; k < NX; ++k)
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+          if (k == 0 || t + k * PB_THREADS < K[1] * K[2]) u[k][j] = c[xsrc[k] + plane[j]];
+    };
+    load(f0);
+#pragma unroll 1
+    for (int f = f0; f < f0 + PB_FIELDS; ++f) {
+#pragma unroll
+      for (int k = 0; k < NX; ++k)
+        if (t + k * PB_THREADS < K[1] * K[2]) {
+#pragma unroll
+          for (int xl = 0; xl < PB_SW; ++xl)
+            if (xl < nx)
+              X[xl * PB_KMAX * PB_KMAX + xdst[k]] =
+                  refine_1d(u[k] + ((ODD + xl) >> 1), 1, (ODD + xl) & 1);
+        }
+      __syncthreads();
+      if (f + 1 < f0 + PB_FIELDS) load(f + 1);     // in flight during the y and z passes
+#pragma unroll
+      for (int k = 0; k < NY; ++k)
+        if (yitem[k] >= 0)
+          Y[(yitem[k] >> 12) & 4095] = refine_1d(X + (yitem[k] & 4095), PB_KMAX, yitem[k] >> 24);
+      __syncthreads();
+      double* out = pool + jb.dst + (long)f * P;
+#pragma unroll
+      for (int k = 0; k < NZ; ++k)
+        if (zitem[k] >= 0)
+          out[(zitem[k] >> 12) & 16383] = refine_1d(Y + (zitem[k] & 4095), 1, zitem[k] >> 26);
+    }
+  };
+  if ((r0[0] + x0) & 1)
+    run(std::integral_constant<int, 1>());
+  else
+    run(std::integral_constant<int, 0>());
 }
+static_assert(PB_SW * PB_KMAX * PB_KMAX <= 4096 && PB_SW * PB_WMAX * PB_KMAX <= 4096 &&
+                  PB_WMAX * PB_WMAX * PB_WMAX <= 16384,
+              "packed items");
 
 hipError_t launch_prolong_blocks(double* pool, long long pool_n, const void* jobs, long n,
                                  hipStream_t st) {
+  constexpr long per_job = (BSSN_NF / PB_FIELDS) * PB_SLABS;
   if (n <= 0) return hipSuccess;
-  if (n > 0x7fffffffL / (BSSN_NF * PB_SLABS)) return hipErrorInvalidValue;   // grid too large
-  hipLaunchKernelGGL(k_prolong_block, dim3((unsigned)(n * BSSN_NF * PB_SLABS)),
-                     dim3(BSSN_PB_THREADS), 0, st, pool, (const bssn_prolong_block*)jobs, pool_n);
+  if (n > 0x7fffffffL / per_job) return hipErrorInvalidValue;   // grid too large
+  hipLaunchKernelGGL(k_prolong_block, dim3((unsigned)(n * per_job)), dim3(PB_THREADS), 0, st,
+                     pool, (const bssn_prolong_block*)jobs, pool_n);
   return hipGetLastError();
 }
 
