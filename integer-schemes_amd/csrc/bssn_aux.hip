@@ -118,11 +118,11 @@ void k_deriv_bundle(const double* __restrict__ F, BundleOut o, Dims d, Scales w)
     const int f = f0 + i, sl = s2slot(f);
     s.stage_in(f, i & 1, i + 1 < kFieldRun ? f + 1 : -1);
 #pragma unroll
-    for (int a = 0; a < 3; ++a) bundle_put<STORE>(o, 3 * f + a, d.P, s.gc, s.d1(a), valid);
+    for (int a = 0; a < 3; ++a) bundle_put<STORE>(o, 3 * f + a, d.P, s.gp, s.d1(a), valid);
     if (sl >= 0) {
 #pragma unroll
       for (int q = 0; q < 6; ++q)
-        bundle_put<STORE>(o, 72 + 6 * sl + q, d.P, s.gc, s.d2(pi_(q), pj_(q)), valid);
+        bundle_put<STORE>(o, 72 + 6 * sl + q, d.P, s.gp, s.d2(pi_(q), pj_(q)), valid);
     }
   }
 }
@@ -359,11 +359,11 @@ __global__ __launch_bounds__(64) void k_ko_add(const double* __restrict__ F,
   // load is in bounds for every lane).
   constexpr int DEPTH = ORD == 4 ? 2 : 1;
   WaveSrc<ORD, true, MODE, StateOrder, DEPTH> s(lds, F, w, d, ox, oy, oz, lane);
-  double o = OUT[s.gc];
+  double o = OUT[s.gp];
   auto field = [&](int f, auto slot) {
     s.template stage_slot<decltype(slot)::value>(f);
     const double k = s.ko();
-    const long i = (long)f * d.P + s.gc;
+    const long i = (long)f * d.P + s.gp;
     if (valid) OUT[i] = o + k;
     if (f + 1 < BSSN_NF) o = OUT[i + d.P];
     __builtin_amdgcn_wave_barrier();

@@ -113,11 +113,11 @@ __device__ __forceinline__ void batch_brick(double* lds, const StageArgs& args,
   using Src = WaveSrc<ORD, KO, MODE, RhsOrder, fused_depth<KIND, ORD>()>;
   if constexpr (MODE == LINK) {
     Src src(lds, args.Yin, B.off, b.link + 2 * blk.moff, b.pool_n, B.w, B.d, ox, oy, oz, lane);
-    StageOut<KIND> out(B.a, B.d.P, src.gc, lane_valid<G>(B.d, ox, oy, oz, lane), true);
+    StageOut<KIND> out(B.a, B.d.P, src.gp, lane_valid<G>(B.d, ox, oy, oz, lane), true);
     bssn_rhs_point<KO>(src, B.sc, out);
   } else {
     Src src(lds, B.a.Yin, B.w, B.d, ox, oy, oz, lane);
-    StageOut<KIND> out(B.a, B.d.P, src.gc, lane_valid<G>(B.d, ox, oy, oz, lane), true);
+    StageOut<KIND> out(B.a, B.d.P, src.gp, lane_valid<G>(B.d, ox, oy, oz, lane), true);
     bssn_rhs_point<KO>(src, B.sc, out);
   }
 }
@@ -164,11 +164,11 @@ void k_fused_batch_group(StageArgs args, BatchArgs b) {
   using Src = GroupSrc<ORD, KO, MODE>;
   if constexpr (MODE == LINK) {
     Src src(mem, args.Yin, B.off, b.link + 2 * blk.moff, b.pool_n, B.w, B.d, ox, oy, oz, t);
-    StageOut<KIND, true> out(B.a, B.d.P, src.gc, lane_valid<G>(B.d, ox, oy, oz, t), true);
+    StageOut<KIND, true> out(B.a, B.d.P, src.gp, lane_valid<G>(B.d, ox, oy, oz, t), true);
     bssn_rhs_point<KO>(src, B.sc, out);
   } else {
     Src src(mem, B.a.Yin, B.w, B.d, ox, oy, oz, t);
-    StageOut<KIND, true> out(B.a, B.d.P, src.gc, lane_valid<G>(B.d, ox, oy, oz, t), true);
+    StageOut<KIND, true> out(B.a, B.d.P, src.gp, lane_valid<G>(B.d, ox, oy, oz, t), true);
     bssn_rhs_point<KO>(src, B.sc, out);
   }
 }

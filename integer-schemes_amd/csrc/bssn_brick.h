@@ -307,14 +307,28 @@ struct BoxStencil {
   }
 };
 
-// halo position -> grid index along one axis (clamped, or wrapped over the interior)
+// halo position -> grid index along one axis (clamped, wrapped over the interior, or both: CARRY,
+// which needs an interior of at least ng points)
 template <int MODE>
 __device__ __forceinline__ int map_axis(int v, int S, int ng) {
-  if (MODE == CLAMP) return v < 0 ? 0 : (v > S - 1 ? S - 1 : v);
+  if (MODE == CLAMP || MODE == CARRY) v = v < 0 ? 0 : (v > S - 1 ? S - 1 : v);
+  if (MODE == CLAMP) return v;
   const int N = S - 2 * ng;
+  if (MODE == CARRY) return v < ng ? v + N : (v >= ng + N ? v - N : v);
   int w = (v - ng) % N;
   w = w < 0 ? w + N : w;
   return ng + w;
+}
+
+// flat index of the point whose value the state holds at the lane's point: its own, or (CARRY)
+// its periodic image
+template <class G, int MODE>
+__device__ __forceinline__ long lane_centre(const Dims& d, int ox, int oy, int oz, int lane) {
+  if (MODE != CARRY) return lane_point<G>(d, ox, oy, oz, lane);
+  const int x = map_axis<CARRY>(ox + G::lx(lane), d.S[0], d.ng);
+  const int y = map_axis<CARRY>(oy + G::ly(lane), d.S[1], d.ng);
+  const int z = map_axis<CARRY>(oz + G::lz(lane), d.S[2], d.ng);
+  return ((long)x * d.S[1] + y) * d.S[2] + z;
 }
 
 // Source of fields and derivatives for bssn_rhs_point: one wave-private LDS box per field.
@@ -337,7 +351,8 @@ struct WaveSrc : BoxStencil<Geo<ORD, KO>, Coef<ORD>> {
   int psrc[MODE == LINK ? G::PER : 1];   // LINK: field stride of each staged cell's block
   int cel[G::PER];      // box indices of this lane's staged cells
   double pf[DEPTH][G::PER];   // the next DEPTH fields' cells, in flight (slot = position % DEPTH)
-  long gc;              // flat index of the lane's point (clamped into the grid)
+  long gp;              // flat index of the lane's point (clamped into the grid)
+  long gc;              // flat index of its centre value (gp, or its periodic image)
   static constexpr bool kEarlyCentres = true;   // bssn_rhs_point: prefetch centres
 
   __device__ __forceinline__ WaveSrc(double* lds_, const double* F_, const Scales& sc_,
@@ -346,7 +361,8 @@ struct WaveSrc : BoxStencil<Geo<ORD, KO>, Coef<ORD>> {
     static_assert(MODE != LINK, "LINK sources take the pool and the link map");
     const int tx = G::lx(lane), ty = G::ly(lane), tz = G::lz(lane);
     c = (tx + G::H) * G::SX + (ty + G::H) * G::SY + (tz + G::H);
-    gc = lane_point<G>(d, ox, oy, oz, lane);
+    gp = lane_point<G>(d, ox, oy, oz, lane);
+    gc = lane_centre<G, MODE>(d, ox, oy, oz, lane);
     const int o[3] = {ox, oy, oz};
 #pragma unroll
     for (int k = 0; k < G::PER; ++k) {
@@ -374,7 +390,8 @@ struct WaveSrc : BoxStencil<Geo<ORD, KO>, Coef<ORD>> {
     static_assert(MODE == LINK, "the link constructor is for LINK sources");
     const int tx = G::lx(lane), ty = G::ly(lane), tz = G::lz(lane);
     c = (tx + G::H) * G::SX + (ty + G::H) * G::SY + (tz + G::H);
-    gc = lane_point<G>(d, ox, oy, oz, lane);
+    gp = lane_point<G>(d, ox, oy, oz, lane);
+    gc = lane_centre<G, MODE>(d, ox, oy, oz, lane);
     const int o[3] = {ox, oy, oz};
 #pragma unroll
     for (int k = 0; k < G::PER; ++k) {

@@ -41,7 +41,7 @@ void k_fused(StageArgs args, Dims d, Scales w, Scal sc) {
   const int lane = (int)threadIdx.x;
   if constexpr (SDEV) args_from_pack<ORD>(args, w, sc);
   WaveSrc<ORD, KO, MODE, RhsOrder, fused_depth<KIND, ORD>()> src(lds, args.Yin, w, d, ox, oy, oz, lane);
-  StageOut<KIND> out(args, d.P, src.gc, lane_valid<G>(d, ox, oy, oz, lane),
+  StageOut<KIND> out(args, d.P, src.gp, lane_valid<G>(d, ox, oy, oz, lane),
                      true);
   bssn_rhs_point<KO>(src, with_ssl(sc, args.tdev, args.toff), out);
 }
@@ -59,7 +59,7 @@ void k_fused_group(StageArgs args, Dims d, Scales w, Scal sc) {
   const int t = (int)threadIdx.x;
   if constexpr (SDEV) args_from_pack<ORD>(args, w, sc);
   GroupSrc<ORD, KO, MODE> src(mem, args.Yin, w, d, ox, oy, oz, t);
-  StageOut<KIND, true> out(args, d.P, src.gc, lane_valid<G>(d, ox, oy, oz, t), true);
+  StageOut<KIND, true> out(args, d.P, src.gp, lane_valid<G>(d, ox, oy, oz, t), true);
   bssn_rhs_point<KO>(src, with_ssl(sc, args.tdev, args.toff), out);
 }
 
@@ -86,16 +86,24 @@ static hipError_t launch_fused_t(const StageArgs& a, const Dims& d, const Scales
   return hipGetLastError();
 }
 
+template <int ORD, bool KO, int KIND, bool SDEV>
+static hipError_t launch_fused_mode(const StageArgs& a, const Dims& d, const Scales& w,
+                                    const Scal& sc, int mode, hipStream_t st) {
+  if (mode == WRAP) return launch_fused_t<ORD, KO, WRAP, KIND, SDEV>(a, d, w, sc, st);
+  if (mode == CLAMP) return launch_fused_t<ORD, KO, CLAMP, KIND, SDEV>(a, d, w, sc, st);
+  if constexpr (KIND != KIND_RHS)   // the carried-ghost steps' stages
+    return launch_fused_t<ORD, KO, CARRY, KIND, SDEV>(a, d, w, sc, st);
+  return hipErrorInvalidValue;
+}
+
 // every (KO, MODE, kind) instance of one FD order with the host pack
 template <int ORD>
 static hipError_t launch_fused_ord(const StageArgs& a, const Dims& d, const Scales& w,
                                    const Scal& sc, bool ko, int mode, hipStream_t st) {
   return with_kind<true>(a.kind, [&](auto k) -> hipError_t {
     constexpr int K = decltype(k)::value;
-    if (ko) return mode == WRAP ? launch_fused_t<ORD, true, WRAP, K, false>(a, d, w, sc, st)
-                                : launch_fused_t<ORD, true, CLAMP, K, false>(a, d, w, sc, st);
-    return mode == WRAP ? launch_fused_t<ORD, false, WRAP, K, false>(a, d, w, sc, st)
-                        : launch_fused_t<ORD, false, CLAMP, K, false>(a, d, w, sc, st);
+    return ko ? launch_fused_mode<ORD, true, K, false>(a, d, w, sc, mode, st)
+              : launch_fused_mode<ORD, false, K, false>(a, d, w, sc, mode, st);
   });
 }
 
@@ -105,10 +113,8 @@ static hipError_t launch_fused_ord_sdev(const StageArgs& a, const Dims& d, const
                                         const Scal& sc, bool ko, int mode, hipStream_t st) {
   return with_kind<false>(a.kind, [&](auto k) -> hipError_t {
     constexpr int K = decltype(k)::value;
-    if (ko) return mode == WRAP ? launch_fused_t<ORD, true, WRAP, K, true>(a, d, w, sc, st)
-                                : launch_fused_t<ORD, true, CLAMP, K, true>(a, d, w, sc, st);
-    return mode == WRAP ? launch_fused_t<ORD, false, WRAP, K, true>(a, d, w, sc, st)
-                        : launch_fused_t<ORD, false, CLAMP, K, true>(a, d, w, sc, st);
+    return ko ? launch_fused_mode<ORD, true, K, true>(a, d, w, sc, mode, st)
+              : launch_fused_mode<ORD, false, K, true>(a, d, w, sc, mode, st);
   });
 }
 

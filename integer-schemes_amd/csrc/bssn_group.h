@@ -95,8 +95,9 @@ struct GroupSrc : BoxStencil<GroupGeo<ORD, KO>, Coef<ORD>> {
   int psrc[MODE == LINK ? G::PER : 1];   // LINK: field stride of each staged cell's block
   int cel[G::PER];      // box indices of this lane's staged cells
   double pf[G::PER];    // the next field's cells, in flight
-  std::conditional_t<WIDE, long, unsigned> gc;   // the lane's point, clamped into the grid: byte
-                                                 // offset in a field (WIDE: index)
+  // the lane's point, clamped into the grid, and the place of its centre value (the point, or its
+  // periodic image): byte offsets in a field (WIDE: indices)
+  std::conditional_t<WIDE, long, unsigned> gp, gc;
   static constexpr int kParkSlots = G::SLOTS;
 
   __device__ __forceinline__ GroupSrc(double* mem, const double* F_, const Scales& sc_,
@@ -157,8 +158,12 @@ struct GroupSrc : BoxStencil<GroupGeo<ORD, KO>, Coef<ORD>> {
 
   __device__ __forceinline__ void place(const Dims& d, int ox, int oy, int oz, int t) {
     c = (G::lx(t) + G::H) * G::SX + (G::ly(t) + G::H) * G::SY + (G::lz(t) + G::H);
-    gc = lane_point<G>(d, ox, oy, oz, t);
-    if constexpr (!WIDE) gc <<= 3;
+    gp = lane_point<G>(d, ox, oy, oz, t);
+    gc = lane_centre<G, MODE>(d, ox, oy, oz, t);
+    if constexpr (!WIDE) {
+      gp <<= 3;
+      gc <<= 3;
+    }
   }
 
   __device__ __forceinline__ static int cells(int f) {

@@ -40,7 +40,10 @@ namespace bssn {
 // LINK (batched blocks only): cells that are ghosts of the block are read where the link map
 // points (a neighbouring block's interior point, or the block's own ghost where a prolongation
 // fills it), so a step needs no ghost copies between its stages.
-enum Mode : int { CLAMP = 0, WRAP = 1, LINK = 2 };
+// CARRY: the values CLAMP would read from a periodically synced copy of the state (halo positions
+// clamped to the padded grid, then ghost positions wrapped into the interior), for points of the
+// whole padded grid.
+enum Mode : int { CLAMP = 0, WRAP = 1, LINK = 2, CARRY = 3 };
 
 enum Field : int {
   ALPHA = 0, CHI = 1, KTR = 2,
