@@ -50,6 +50,10 @@ __device__ __forceinline__ void out_phase(Out&) {}
 template <class Out>
 __device__ __forceinline__ void out_prep(Out&, int) {}
 
+// source hook between the Ricci tensor's metric part and the chi phase: nothing by default
+template <class Src>
+__device__ __forceinline__ void after_ricci(Src&) {}
+
 template <class S, class = void>
 struct ParkSlots : std::integral_constant<int, 0> {};
 template <class S>
@@ -260,6 +264,7 @@ __device__ __forceinline__ void bssn_rhs_point(Src& s, const Scal& P, Out& o) {
 
   if constexpr (PK > 0) {
     __builtin_amdgcn_sched_barrier(0);
+    after_ricci(s);
 #pragma unroll
     for (int q = 0; q < 6; ++q) g[q] = kept(P_RA + q);
 #pragma unroll
@@ -537,10 +542,12 @@ __device__ __forceinline__ void bssn_constraints_point(Src& s, Out& o) {
   }
   ricci_metric(dg, ig, C2, CalGt, Rt);
   if constexpr (PARK) {
+#pragma unroll
+    for (int q = 0; q < 6; ++q) BSSN_PIN(Rt[q]);
     __builtin_amdgcn_sched_barrier(0);
+    after_ricci(s);
 #pragma unroll
     for (int q = 0; q < 6; ++q) {
-      BSSN_PIN(Rt[q]);
       g[q] = s.parked(q);
     }
   }

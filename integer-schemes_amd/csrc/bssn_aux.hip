@@ -91,13 +91,13 @@ __device__ __forceinline__ void bundle_put(const BundleOut& o, int slot, long P,
   }
 }
 
-// Bricks shared by four waves, two boxes, a barrier per field (bssn_group.h), kFieldRun fields per
+// Bricks shared by four waves (bssn_group.h), kFieldRun fields per
 // workgroup (blockIdx.y). What bounds the pass is the store of the 138 arrays (with the stencils
 // left out it takes as long): 4 x 4 x 16 bricks write rows of 128 B, where a wave's own 4 x 4 x 4
 // brick wrote pieces of 32 B, and the runs, dispatched one after the other, write 3 to 18 arrays
 // at a time instead of 138. 134^3, FD6 fp64 / 118^3, FD4 BFP32: 2.08 / 0.96 -> 1.33 / 0.50 ms (runs
 // of 1 / 3 / 4 / 8 / 24 fields: 1.38 / 1.35 / 1.37 / 1.43 / 1.48 and 0.53 / 0.50 / 0.51 / 0.51 /
-// 0.54). Rows that start on a 128 B line write a quarter faster (2.85 against 2.13 TB/s); the
+// 0.54); with the shared numerators FD6 1.29, 134^3 FD4 fp64 1.25 -> 1.14 ms. Rows that start on a 128 B line write a quarter faster (2.85 against 2.13 TB/s); the
 // caller's row pitch decides that.
 constexpr int kFieldRun = 2;
 static_assert(BSSN_NF % kFieldRun == 0, "whole runs");
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(ORD == 8 ? 2 : 4)))
 void k_deriv_bundle(const double* __restrict__ F, BundleOut o, Dims d, Scales w) {
   using G = GroupGeo<ORD, false>;
-  __shared__ double mem[2 * G::VOL];
+  __shared__ double mem[G::BOX_DOUBLES];
   int ox, oy, oz;
   if (!brick_origin<G>(d, &ox, &oy, &oz)) return;
   const int t = (int)threadIdx.x, f0 = (int)blockIdx.y * kFieldRun;
@@ -116,7 +116,7 @@ void k_deriv_bundle(const double* __restrict__ F, BundleOut o, Dims d, Scales w)
 #pragma unroll 1
   for (int i = 0; i < kFieldRun; ++i) {
     const int f = f0 + i, sl = s2slot(f);
-    s.stage_in(f, i & 1, i + 1 < kFieldRun ? f + 1 : -1);
+    s.stage_in(f, i + 1 < kFieldRun ? f + 1 : -1);
 #pragma unroll
     for (int a = 0; a < 3; ++a) bundle_put<STORE>(o, 3 * f + a, d.P, s.gp, s.d1(a), valid);
     if (sl >= 0) {
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(256) void k_bundle_absmax(const double* __restrict_
                                                        unsigned long long* __restrict__ amax,
                                                        Dims d, Scales w) {
   using G = GroupGeo<ORD, false>;
-  __shared__ double mem[2 * G::VOL];
+  __shared__ double mem[G::BOX_DOUBLES];
   constexpr int NA = EDGES ? 9 : 3;   // arrays of the field
   const int t = (int)threadIdx.x, y = (int)blockIdx.y;
   const int f = EDGES ? (y < KTR ? y : y + 1) : (y == 0 ? KTR : AT0 - 1 + y);
@@ -179,14 +179,13 @@ __global__ __launch_bounds__(256) void k_bundle_absmax(const double* __restrict_
             nbz = (d.n[2] + G::BZ - 1) / G::BZ;
   const int nb = nbx * nby * nbz;
   double m[NA] = {};
-  int box = 0;
-  for (int L = (int)blockIdx.x; L < nb; L += (int)gridDim.x, box ^= 1) {
+  for (int L = (int)blockIdx.x; L < nb; L += (int)gridDim.x) {
     const int bz = L % nbz, c = L / nbz, by = c % nby, bx = c / nby;
     const int ox = d.lo[0] + bx * G::BX, oy = d.lo[1] + by * G::BY, oz = d.lo[2] + bz * G::BZ;
     const bool valid = lane_valid<G>(d, ox, oy, oz, t);
     GroupSrc<ORD, false, CLAMP, OneField<EDGES>, WIDE> s(mem, F + (long)f * d.P, w, d, ox, oy,
                                                          oz, t);
-    s.stage_in(0, box, -1);   // the boxes alternate from brick to brick
+    s.stage_in(0, -1);
 #pragma unroll
     for (int a = 0; a < 3; ++a) m[a] = nanmax_d(m[a], valid ? fabs(s.d1(a)) : 0.0);
     if constexpr (EDGES) {
@@ -487,7 +486,7 @@ __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(2, 2)))
 void k_constraints(const double* __restrict__ F, double* __restrict__ HM, Dims d, Scales w) {
   using G = GroupGeo<ORD, false>;
-  __shared__ double mem[2 * G::VOL + 6 * G::NT];   // two boxes and six parked values per lane
+  __shared__ double mem[G::BOX_DOUBLES + 6 * G::NT];   // six parked values per lane
   int ox, oy, oz;
   if (!brick_origin<G>(d, &ox, &oy, &oz)) return;
   const int t = (int)threadIdx.x;

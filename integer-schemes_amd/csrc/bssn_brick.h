@@ -260,25 +260,28 @@ struct BoxStencil {
     return a == 0 ? G::SX : (a == 1 ? G::SY : 1);
   }
 
-  // unscaled first-derivative numerator along axis a at box index q
-  __device__ __forceinline__ double n1(int q, int a) const {
-    const int s = stride(a);
+  // unscaled first-derivative numerator at box index q along the axis of stride s, along axis a
+  __device__ __forceinline__ double n1s(int q, int s) const {
     double acc = 0.0;
 #pragma unroll
     for (int k = 1; k <= G::R; ++k) acc += C::d1(k) * (lds[q + k * s] - lds[q - k * s]);
+    return acc;
+  }
+  __device__ __forceinline__ double n1(int q, int a) const { return n1s(q, stride(a)); }
+
+  // unscaled second-derivative numerator along axis a at the point
+  __device__ __forceinline__ double n2(int a) const {
+    const int s = stride(a);
+    double acc = C::d2(0) * lds[c];
+#pragma unroll
+    for (int k = 1; k <= G::R; ++k) acc += C::d2(k) * (lds[c + k * s] + lds[c - k * s]);
     return acc;
   }
 
   __device__ __forceinline__ double d1(int a) const { return pin(n1(c, a) * sc.s1[a]); }
 
   __device__ __forceinline__ double d2(int i, int j) const {
-    if (i == j) {
-      const int s = stride(i);
-      double acc = C::d2(0) * lds[c];
-#pragma unroll
-      for (int k = 1; k <= G::R; ++k) acc += C::d2(k) * (lds[c + k * s] + lds[c - k * s]);
-      return pin(acc * sc.s2[i]);
-    }
+    if (i == j) return pin(n2(i) * sc.s2[i]);
     const int sj = stride(j);
     double acc = 0.0;
 #pragma unroll

@@ -202,6 +202,10 @@ __device__ __forceinline__ double pin(double x) {
   asm volatile("" : "+v"(x));
   return x;
 }
+__device__ __forceinline__ int pin(int x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
 #endif
 
 }  // namespace bssn
