@@ -13,12 +13,16 @@
 //   box values v -> c = 0.5 max + 0.5 min (stencils annihilate constants), sigma = 2^(6-E) with
 //   max|v - c| = f 2^E, r0 = (v - c) sigma, q_s = rint(r_s), r_{s+1} = 128 (r_s - q_s):
 //   |q_s| <= 64, every step exact; (v - c) sigma = sum_s q_s 2^(-7 s) + O(2^(-7 k)).
-//   Per digit plane q_s (int8, 32 x 32):
-//     B q   (rows: outputs along axis 1)   = v_mfma_i32_32x32x32_i8(band, q)
-//     q B^T (columns: outputs along axis 2) = v_mfma_i32_32x32x32_i8(q^T via LDS, band)
-//     B q B^T (mixed): the INT32 B q is split into two int8 digits (|B q| <= 18 * 64) and each
-//           is multiplied by B^T, so the mixed contraction is exact too.
-//   Recombination in FP64: acc += P_s 2^(-7 s) (exact terms), D = (acc 2^-e) * scale.
+//   The k <= 7 digits are taken in three groups (0..2, 3..5, 6), each as one integer
+//   N = rint(r 2^(7 (g - 1))) = sum_s q_s 2^(7 (g - 1 - s)) (g digits; the remainder is the same,
+//   and a tie falls the same way), whose signed bytes are the int8 operands (32 x 32 planes):
+//     B N   (rows: outputs along axis 1)   = sum of v_mfma_i32_32x32x32_i8(band, byte plane)
+//     N B^T (columns: outputs along axis 2) = the same with N^T, transposed as words via LDS
+//     B N B^T (mixed): the INT32 B N (25 bits and sign) in its four signed bytes, each times B^T
+//   INT32 holds every exact result (the mixed one: 18 * 18 * 64 * 2^14.02 < 2^29).
+//   Recombination in FP64: acc += P_g 2^(-7 s), s the group's last digit; D = (acc 2^-e) * scale.
+//   The sums of digits 0..5 are exact in FP64 (at most 15 + 35 bits), so the only rounding is
+//   that of digit 6, as if the digits had been added one by one.
 // The integer stencils are those of common/src/mcs_common/derivatives.py:33-49 times 12
 // (first and second derivatives) and 144 (mixed).
 //
@@ -27,6 +31,8 @@
 #include <hip/hip_runtime.h>
 
 #include <math.h>
+
+#include <type_traits>
 
 #include "bssn_kernels.h"
 #include "bssn_params.h"
@@ -68,11 +74,65 @@ __device__ __forceinline__ v4i band_operand(int lane) {
   return v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
 }
 
-__device__ __forceinline__ v4i pack16(const int* q) {
-  unsigned w[4] = {0u, 0u, 0u, 0u};
+// Byte planes of 16 words: plane b holds byte b of each, in order.
+template <int NP>
+__device__ __forceinline__ void byte_planes(const int* w, v4i* plane) {
 #pragma unroll
-  for (int j = 0; j < 16; ++j) w[j >> 2] |= ((unsigned)q[j] & 0xffu) << (8 * (j & 3));
-  return v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+  for (int g = 0; g < 4; ++g) {
+    const int* a = w + 4 * g;
+    const unsigned lo01 = __builtin_amdgcn_perm(a[1], a[0], 0x05010400u);
+    const unsigned lo23 = __builtin_amdgcn_perm(a[3], a[2], 0x05010400u);
+    plane[0][g] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
+    if constexpr (NP > 1) plane[1][g] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
+    if constexpr (NP > 2) {
+      const unsigned hi01 = __builtin_amdgcn_perm(a[1], a[0], 0x07030602u);
+      const unsigned hi23 = __builtin_amdgcn_perm(a[3], a[2], 0x07030602u);
+      plane[2][g] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
+      if constexpr (NP > 3) plane[3][g] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
+    }
+  }
+}
+
+// v as NP signed bytes: v = sum_b byte_b 256^b (|v| < 2^(8 NP - 1) - 2^(8 NP - 8))
+template <int NP>
+__device__ __forceinline__ int signed_bytes(int v) {
+  constexpr int h = NP == 1 ? 0 : (NP == 2 ? 0x80 : (NP == 3 ? 0x8080 : 0x808080));
+  return (v + h) ^ h;
+}
+
+// The contraction of a matrix of signed bytes (NP planes) with the band: rows (band times the
+// matrix, planes in the B distribution) or columns (the matrix times band^T, A distribution).
+template <int NP, bool ROWS>
+__device__ __forceinline__ v16i contract(const v4i& band, const v4i* plane) {
+  const v16i z16 = {};
+  v16i sum = z16;
+#pragma unroll
+  for (int b = NP - 1; b >= 0; --b) {
+    const v16i p = ROWS ? __builtin_amdgcn_mfma_i32_32x32x32_i8(band, plane[b], z16, 0, 0, 0)
+                        : __builtin_amdgcn_mfma_i32_32x32x32_i8(plane[b], band, z16, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 16; ++i)   // the partial sums may wrap, the result does not
+      sum[i] = b == NP - 1 ? p[i] : (int)(((unsigned)sum[i] << 8) + (unsigned)p[i]);
+  }
+  return sum;
+}
+
+typedef v4i __attribute__((may_alias)) v4i_lds;
+// 32 x 32 words; the rows' starts, 36 words apart, lie on 16 different groups of 4 banks
+constexpr int I8_PITCH = 36;
+
+// row r = lane % 32, positions 16 (lane / 32) + j of the words in t, as byte planes
+template <int NP>
+__device__ __forceinline__ void row_planes(const int* t, int lane, v4i* plane) {
+  int w[16];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const v4i x = *(const v4i_lds*)&t[(lane & 31) * I8_PITCH + 16 * (lane >> 5) + 4 * g];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[4 * g + j] = x[j];
+  }
+  __builtin_amdgcn_wave_barrier();
+  byte_planes<NP>(w, plane);
 }
 
 __device__ __forceinline__ double wave_max(double x) {
@@ -114,8 +174,7 @@ __host__ __device__ inline long i8_tiles(const int* S) {
 // TWO: the fields with second derivatives (else first derivatives only).
 // One wave: tile w (plane fastest, then tile along axis 2, along axis 1, field) of the grid a.
 template <int ORIENT, bool TWO>
-__device__ __forceinline__ void i8_tile(const I8Args& a, long w, int lane, signed char* tq,
-                                        signed char* th, signed char* tl) {
+__device__ __forceinline__ void i8_tile(const I8Args& a, long w, int lane, int* t) {
   constexpr int AX1 = ORIENT == 0 ? 1 : 0;
   constexpr int AX2 = ORIENT == 2 ? 1 : 2;
   constexpr int AXP = ORIENT == 0 ? 0 : (ORIENT == 1 ? 1 : 2);
@@ -129,12 +188,25 @@ __device__ __forceinline__ void i8_tile(const I8Args& a, long w, int lane, signe
   const int n1 = a.S[AX1], n2 = a.S[AX2], npl = a.S[AXP];
   const long st[3] = {(long)a.S[1] * a.S[2], (long)a.S[2], 1L};
   const int nt1 = (n1 + I8_TILE - 1) / I8_TILE, nt2 = (n2 + I8_TILE - 1) / I8_TILE;
-  const int pl = (int)(w % npl);
-  w /= npl;
-  const int t2 = (int)(w % nt2);
-  w /= nt2;
-  const int t1 = (int)(w % nt1);
-  const int fi = (int)(w / nt1);
+  // (y, z) and (x, z) planes: tiles along z fastest, so the lines that two of them share are
+  // complete before they leave L2; (x, y) planes: planes (along z) fastest
+  int pl, t1, t2;
+  if constexpr (ORIENT == 2) {
+    pl = (int)(w % npl);
+    w /= npl;
+    t2 = (int)(w % nt2);
+    w /= nt2;
+    t1 = (int)(w % nt1);
+    w /= nt1;
+  } else {
+    t2 = (int)(w % nt2);
+    w /= nt2;
+    t1 = (int)(w % nt1);
+    w /= nt1;
+    pl = (int)(w % npl);
+    w /= npl;
+  }
+  const int fi = (int)w;
   if (fi >= NF) return;
   const int f = TWO ? kTwoFields[fi] : kOneFields[fi];
   const int o1 = t1 * I8_TILE, o2 = t2 * I8_TILE;
@@ -173,73 +245,50 @@ __device__ __forceinline__ void i8_tile(const I8Args& a, long w, int lane, signe
 #pragma unroll
   for (int j = 0; j < 16; ++j) r[j] = ldexp(r[j], e);
 
-  const v4i band1 = band_operand<1>(lane);
-  const v4i band2 = band_operand<2>(lane);
-  double acc1a[16], acc2a[16], acc1b[16], acc2b[16], accm[16];
+  if (m == INFINITY) {   // infinities have no digits: what the saturating conversion leaves
 #pragma unroll
-  for (int i = 0; i < 16; ++i) acc1a[i] = acc2a[i] = acc1b[i] = acc2b[i] = accm[i] = 0.0;
+    for (int j = 0; j < 16; ++j) r[j] = r[j] == INFINITY ? -1.0 : 0.0;
+  }
 
-  for (int s = 0; s < a.nslice; ++s) {
-    int q[16];
+  // digits 0..na-1, na..na+nb-1 and 6
+  const int ns = a.nslice, na = ns < 3 ? ns : 3, nb = ns < 6 ? ns - na : 3;
+  const bool more = ns > 3, last = ns > 6;
+  v4i qa[3], qb[3], qc[1], ta[3], tb[3], tc[1];   // byte planes of N and of N^T
+  constexpr bool COLS = D1B || D2B;
+  auto digits = [&](auto np, int g, v4i* q, v4i* tr) {
+    constexpr int NP = decltype(np)::value;
+    const double up = ldexp(1.0, 7 * (g - 1));
+    int n[16];
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
-      const double d = rint(r[j]);
-      q[j] = (int)d;
-      r[j] = (r[j] - d) * 128.0;
+      const double x = r[j] * up, d = rint(x);
+      r[j] = (x - d) * 128.0;
+      n[j] = signed_bytes<NP>((int)d);
     }
-    const double ws = ldexp(1.0, -7 * s);
-    const v4i qb = pack16(q);
-    const v16i z16 = {};
-    v16i p1 = z16;
-    if (D1A || MIX) p1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(band1, qb, z16, 0, 0, 0);
-    if (D2A) {
-      const v16i p2 = __builtin_amdgcn_mfma_i32_32x32x32_i8(band2, qb, z16, 0, 0, 0);
+    byte_planes<NP>(n, q);
+    if constexpr (COLS) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc2a[i] = acc2a[i] + (double)p2[i] * ws;
-    }
-    if (D1A) {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc1a[i] = acc1a[i] + (double)p1[i] * ws;
-    }
-    if (D1B || D2B) {
-      // q^T in the A distribution: row = lane % 32 (axis 1), positions along axis 2
-#pragma unroll
-      for (int j = 0; j < 16; ++j) tq[(16 * hh + j) * I8_BOX + c] = (signed char)q[j];
+      for (int j = 0; j < 16; ++j) t[(16 * hh + j) * I8_PITCH + c] = n[j];
       __builtin_amdgcn_wave_barrier();
-      const v4i qa = *(const v4i*)&tq[c * I8_BOX + 16 * hh];
-      __builtin_amdgcn_wave_barrier();
-      if (D1B) {
-        const v16i p = __builtin_amdgcn_mfma_i32_32x32x32_i8(qa, band1, z16, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc1b[i] = acc1b[i] + (double)p[i] * ws;
-      }
-      if (D2B) {
-        const v16i p = __builtin_amdgcn_mfma_i32_32x32x32_i8(qa, band2, z16, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc2b[i] = acc2b[i] + (double)p[i] * ws;
-      }
+      row_planes<NP>(t, lane, tr);
     }
-    if (MIX) {
-      // B q (INT32, |.| <= 18 * 64) as two int8 digits hi * 128 + lo, each times B^T
+  };
+  digits(std::integral_constant<int, 3>(), na, qa, ta);
+  if (more) digits(std::integral_constant<int, 3>(), nb, qb, tb);
+  if (last) digits(std::integral_constant<int, 1>(), 1, qc, tc);
+  const double wa = ldexp(1.0, -7 * (na - 1)), wb = ldexp(1.0, -7 * (na + nb - 1)),
+               wc = ldexp(1.0, -42);
+  double acc[16];
+  auto add = [&](const v16i& p, double ws) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int v = p1[i];
-        const int lo = ((v + 64) & 127) - 64;
-        const int hi = (v - lo) >> 7;
-        const int rr = row_of(i, lane);
-        th[rr * I8_BOX + c] = (signed char)hi;
-        tl[rr * I8_BOX + c] = (signed char)lo;
-      }
-      __builtin_amdgcn_wave_barrier();
-      const v4i ah = *(const v4i*)&th[c * I8_BOX + 16 * hh];
-      const v4i al = *(const v4i*)&tl[c * I8_BOX + 16 * hh];
-      __builtin_amdgcn_wave_barrier();
-      const v16i mh = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah, band1, z16, 0, 0, 0);
-      const v16i ml = __builtin_amdgcn_mfma_i32_32x32x32_i8(al, band1, z16, 0, 0, 0);
+    for (int i = 0; i < 16; ++i) acc[i] = acc[i] + (double)p[i] * ws;
+  };
+  auto clear = [&]() {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) accm[i] = accm[i] + (double)(mh[i] * 128 + ml[i]) * ws;
-    }
-  }
+    for (int i = 0; i < 16; ++i) acc[i] = 0.0;
+  };
+  const v4i band1 = band_operand<1>(lane);
+  const v4i band2 = band_operand<2>(lane);
 
   // outputs: rows along axis 1, columns along axis 2 (lane's column c, rows row_of(i))
   double* Dp = a.D;
@@ -258,21 +307,57 @@ __device__ __forceinline__ void i8_tile(const I8Args& a, long w, int lane, signe
     }
   };
   const int slot = TWO ? fi : -1;
-  if (D1A) put(3 * f + AX1, acc1a, a.s1[AX1], true, false);
-  if (D2A) put(72 + 6 * slot + (AX1 == 0 ? 0 : 3), acc2a, a.s2[AX1], true, false);
-  if (D1B) put(3 * f + AX2, acc1b, a.s1[AX2], false, true);
-  if (D2B) put(72 + 6 * slot + 5, acc2b, a.s2[AX2], false, true);
-  if (MIX) {
+  auto columns = [&](const v4i& band) {
+    clear();
+    add(contract<3, false>(band, ta), wa);
+    if (more) add(contract<3, false>(band, tb), wb);
+    if (last) add(contract<1, false>(band, tc), wc);
+  };
+  if constexpr (D1B) {
+    columns(band1);
+    put(3 * f + AX2, acc, a.s1[AX2], false, true);
+  }
+  if constexpr (D2B) {
+    columns(band2);
+    put(72 + 6 * slot + 5, acc, a.s2[AX2], false, true);
+  }
+  auto rows = [&](const v4i& band) {
+    clear();
+    add(contract<3, true>(band, qa), wa);
+    if (more) add(contract<3, true>(band, qb), wb);
+    if (last) add(contract<1, true>(band, qc), wc);
+  };
+  if constexpr (D1A) {
+    rows(band1);
+    put(3 * f + AX1, acc, a.s1[AX1], true, false);
+  }
+  if constexpr (D2A) {
+    rows(band2);
+    put(72 + 6 * slot + (AX1 == 0 ? 0 : 3), acc, a.s2[AX1], true, false);
+  }
+  if constexpr (MIX) {
+    // B N as signed bytes through LDS (forming it again costs less than keeping it)
+    auto mixed = [&](auto np, const v16i& p, double ws) {
+      constexpr int NP = decltype(np)::value;
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        t[row_of(i, lane) * I8_PITCH + c] = signed_bytes<NP>(p[i]);
+      __builtin_amdgcn_wave_barrier();
+      v4i pl[NP];
+      row_planes<NP>(t, lane, pl);
+      add(contract<NP, false>(band1, pl), ws);
+    };
+    clear();
+    mixed(std::integral_constant<int, 4>(), contract<3, true>(band1, qa), wa);
+    if (more) mixed(std::integral_constant<int, 4>(), contract<3, true>(band1, qb), wb);
+    if (last) mixed(std::integral_constant<int, 2>(), contract<1, true>(band1, qc), wc);
     // pair index of (AX1, AX2): xy 1, xz 2, yz 4; scale index AX1 + AX2 - 1
     const int pair = AX1 == 0 ? (AX2 == 1 ? 1 : 2) : 4;
-    put(72 + 6 * slot + pair, accm, a.sm[AX1 + AX2 - 1], true, true);
+    put(72 + 6 * slot + pair, acc, a.sm[AX1 + AX2 - 1], true, true);
   }
 }
 
-#define BSSN_I8_LDS                                                          \
-  __shared__ __attribute__((aligned(16))) signed char tq[I8_BOX * I8_BOX];   \
-  __shared__ __attribute__((aligned(16))) signed char th[I8_BOX * I8_BOX];   \
-  __shared__ __attribute__((aligned(16))) signed char tl[I8_BOX * I8_BOX]
+#define BSSN_I8_LDS __shared__ __attribute__((aligned(16))) int t[I8_BOX * I8_PITCH]
 
 // Workgroup -> tile, XCD-aware: the dispatcher deals workgroups round-robin over the 8 XCDs;
 // remap so that each XCD takes a contiguous run of tiles (consecutive planes), whose loads and
@@ -285,10 +370,20 @@ __device__ __forceinline__ long xcd_tile() {
   return (w & 7) * (G8 >> 3) + (w >> 3);
 }
 
+// What bounds the passes is the stores, rows of 28 doubles that start anywhere in a line, and the
+// waits at two waves per SIMD. Taking the digits in groups of three (a third of the FP64
+// conversions and sums, words instead of bytes through LDS, for 45 instead of 42 matrix products) and one output array at a time (16 sums live instead of 80: two
+// waves per SIMD instead of one) took the five passes of a 166^3 state from 3.5 to 3.0 ms; the
+// order of the tiles (i8_tile) from 3.0 to 2.6 ms: (y, z) planes 0.89 -> 0.70 and 0.51 -> 0.38, (x, z)
+// planes 0.62 -> 0.57 and 0.34 -> 0.31, (x, y) planes 0.64 ms. Three or four waves per SIMD
+// spill where second derivatives are taken (0.70 -> 0.85 and 1.11 ms); the first-derivative pass on
+// (x, z) planes has the room for four (0.31 -> 0.26 ms).
 template <int ORIENT, bool TWO>
-__global__ __launch_bounds__(64) void k_i8_plane(I8Args a) {
+__global__ __launch_bounds__(64)
+__attribute__((amdgpu_waves_per_eu(ORIENT == 1 && !TWO ? 4 : 1)))
+void k_i8_plane(I8Args a) {
   BSSN_I8_LDS;
-  i8_tile<ORIENT, TWO>(a, xcd_tile(), (int)threadIdx.x, tq, th, tl);
+  i8_tile<ORIENT, TWO>(a, xcd_tile(), (int)threadIdx.x, t);
 }
 
 // The same pass over every block of a batch: block b owns wave tiles [pre[b], pre[b + 1]) of
@@ -322,7 +417,7 @@ __global__ __launch_bounds__(64) void k_i8_plane_batch(const double* pool, doubl
     a.sm[i] = uniform(sc.sm[i]);
   }
   a.nslice = nslice;
-  i8_tile<ORIENT, TWO>(a, (long)(w - pre[b]), (int)threadIdx.x, tq, th, tl);
+  i8_tile<ORIENT, TWO>(a, (long)(w - pre[b]), (int)threadIdx.x, t);
 }
 
 template <int ORIENT, bool TWO>
