@@ -12,7 +12,9 @@ bricks (BSSN_BRICK_TILE_XY: z columns in square tiles of columns, or 0 for rows 
 evaluated (BSSN_STAGE_DEPTH for the RK/MSRK stage kernels, BSSN_RHS_DEPTH for the bare RHS),
 how many algebra phases ahead of its store a field's write-back operands are loaded
 (BSSN_WB_LEAD), and how many waves per SIMD the register allocator targets (BSSN_STAGE_WAVES,
-BSSN_RHS_WAVES; two waves force one field in flight). A knob moves loads, LDS addresses and
+BSSN_RHS_WAVES; two waves force one field in flight). These are knobs of the wave-private kernels:
+grids of up to 1024 of their bricks (--n 40 and below) and the batches' remainders; larger grids
+run on bricks shared by four waves (bssn_group.h), which only BSSN_BRICK_TILE_XY reaches. A knob moves loads, LDS addresses and
 register allocation, not arithmetic, so every variant computes the same RHS.
 
 For every candidate the tuner

@@ -372,12 +372,13 @@ __device__ __forceinline__ long xcd_tile() {
 
 // What bounds the passes is the stores, rows of 28 doubles that start anywhere in a line, and the
 // waits at two waves per SIMD. Taking the digits in groups of three (a third of the FP64
-// conversions and sums, words instead of bytes through LDS, for 45 instead of 42 matrix products) and one output array at a time (16 sums live instead of 80: two
-// waves per SIMD instead of one) took the five passes of a 166^3 state from 3.5 to 3.0 ms; the
-// order of the tiles (i8_tile) from 3.0 to 2.6 ms: (y, z) planes 0.89 -> 0.70 and 0.51 -> 0.38, (x, z)
-// planes 0.62 -> 0.57 and 0.34 -> 0.31, (x, y) planes 0.64 ms. Three or four waves per SIMD
-// spill where second derivatives are taken (0.70 -> 0.85 and 1.11 ms); the first-derivative pass on
-// (x, z) planes has the room for four (0.31 -> 0.26 ms).
+// conversions and sums, words instead of bytes through LDS, for 45 instead of 42 matrix products)
+// and one output array at a time (16 sums live instead of 80: two waves per SIMD instead of one)
+// took the five passes of a 166^3 state from 3.5 to 3.0 ms, the order of the tiles (i8_tile) from
+// 3.0 to 2.6 ms: (y, z) planes 0.89 -> 0.70 and 0.51 -> 0.38, (x, z) planes 0.62 -> 0.57 and
+// 0.34 -> 0.31, (x, y) planes 0.64 ms. Three or four waves per SIMD spill where second derivatives
+// are taken (0.70 -> 0.85 and 1.11 ms); the first-derivative pass on (x, z) planes has the room
+// for four (0.31 -> 0.26 ms).
 template <int ORIENT, bool TWO>
 __global__ __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(ORIENT == 1 && !TWO ? 4 : 1)))
