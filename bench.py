@@ -769,7 +769,7 @@ def main() -> int:
         roof = {"bound": "mfma", "achieved": round(flops_launch / t_launch / 1e12, 3),
                 "peak": PEAK_FP64 / 1e12, "unit": "TFLOP/s", "frac": round(fp64_frac, 4)}
     roof["traffic"] = measured_traffic(f"bssn_rk4_step_{N}^3_fp64_bl_binary")
-    roof["kernel"] = "k_fused<4,KO,WRAP> (RK4 stage)"
+    roof["kernel"] = "k_fused_group<4,KO,WRAP> (RK4 stage)"
     roof["fp64_frac"] = round(fp64_frac, 4)
     roof["hbm_frac"] = round(hbm_frac, 4)
     roof["ms_per_launch"] = round(ms_stage, 4)
