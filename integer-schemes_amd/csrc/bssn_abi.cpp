@@ -12,6 +12,7 @@
 #include <string>
 #include <vector>
 
+#include "bssn_dispatch.h"
 #include "bssn_kernels.h"
 #include "bssn_params.h"
 
@@ -638,7 +639,7 @@ struct bssn_batch {
   int grid_full = 0, grid_inner = 0, grid_ghost = 0;   // one workgroup per brick
   BrickList sfull{}, sinner{};       // the same points in bricks shared by four waves
   int grid_sfull = 0, grid_sinner = 0;
-  bool shared_full = false, shared_inner = false;   // which of the two a launch takes
+  bool small = false;                // every block's fields below 4 GiB, as the shared form needs
   int* ctr = nullptr;                // device queue counters
   int persistent = 0;                // 0, or the persistent wave count
   const long long* i8pre = nullptr;  // device: 5 prefix arrays of the INT8 bundle passes
@@ -726,20 +727,6 @@ std::vector<BrickItem> chunked(const std::vector<std::vector<BrickItem>>& per_bl
   return out;
 }
 
-// Whether a launch over `points` takes the shared bricks: more wave-private bricks than the chip
-// holds at once (one per SIMD, 4 x 256; below that a launch is one brick's latency long, and the
-// wave-private one's is the shorter), fields below 4 GiB (32-bit byte offsets), and enough of the
-// shared bricks' lanes with a point (a block extent of 8 or 24 along z leaves half a brick
-// empty). FD4, blocks of 16 x 16 x n: RK4 step (interiors) at n = 8 / 12 / 16 / 20 / 24 / 32,
-// fill 0.5 / 0.75 / 1 / 0.63 / 0.75 / 1: wave-private 1.83 / 2.63 / 3.51 / 2.81 / 3.26 / 3.20,
-// shared 1.91 / 2.22 / 2.60 / 2.50 / 2.65 / 2.25 ms; RHS (padded) of 16 x 16 x 12 / 16 x 16 x 16
-// blocks, fill 0.47 / 0.58: 1.03 / 1.24 against 1.16 / 1.17 ms.
-constexpr double kSharedFill = 0.55;
-bool take_shared(long wave_bricks, long shared_bricks, long long points, long long largest) {
-  const double lanes = (double)(BSSN_GROUP_X * BSSN_GROUP_Y * BSSN_GROUP_Z) * shared_bricks;
-  return wave_bricks > 4 * 256 && largest < (1LL << 29) && (double)points >= kSharedFill * lanes;
-}
-
 int flat_grid(const int* cb) {
   int mx = 0;
   for (int c = 0; c < BATCH_CHUNKS; ++c) mx = std::max(mx, cb[c + 1] - cb[c]);
@@ -791,8 +778,6 @@ BatchArgs batch_args(const bssn_batch* b, bool interior, const double* S16, doub
   BatchArgs a{};
   a.blk = b->blk;
   a.persistent = b->persistent;
-  a.shared = !b->persistent && (interior ? b->shared_inner : b->shared_full);
-  a.list = a.shared ? (interior ? b->sinner : b->sfull) : (interior ? b->inner : b->full);
   a.ctr = b->ctr;
   a.interior = interior ? 1 : 0;
   a.base = make_scal(S16, dt, t);
@@ -802,8 +787,15 @@ BatchArgs batch_args(const bssn_batch* b, bool interior, const double* S16, doub
   return a;
 }
 
-int run_batch(const bssn_batch* b, const StageArgs& s, const BatchArgs& a, int ord, bool ko,
-              int mode, hipStream_t st) {
+int run_batch(const bssn_batch* b, const StageArgs& s, BatchArgs a, int ord, bool ko, int mode,
+              hipStream_t st) {
+  const BrickList& waves = a.interior ? b->inner : b->full;
+  const BrickList& groups = a.interior ? b->sinner : b->sfull;
+  // a list's brick count is the end of its last chunk
+  a.shared = !b->persistent && b->small &&
+             fused_shared(ord, s.kind == KIND_RHS, ko, true, waves.cb[BATCH_CHUNKS],
+                          groups.cb[BATCH_CHUNKS]);
+  a.list = a.shared ? groups : waves;
   int grid = a.interior ? b->grid_inner : b->grid_full;
   if (a.shared) grid = a.interior ? b->grid_sinner : b->grid_sfull;
   if (b->persistent) {
@@ -903,10 +895,7 @@ int bssn_batch_create(bssn_batch** out, void* plan, size_t plan_bytes, int nblk,
     for (int i = 0; i <= BATCH_CHUNKS; ++i) to[k]->cb[i] = cb[k][i];
     *grid[k] = flat_grid(cb[k]);
   }
-  bt->shared_full = take_shared((long)list[L_FULL].size(), (long)list[L_SFULL].size(), padded,
-                                largest);
-  bt->shared_inner = take_shared((long)list[L_INNER].size(), (long)list[L_SINNER].size(),
-                                 interior, largest);
+  bt->small = largest < kGroupPoints;
   bt->ctr = (int*)(base + o_ctr);
   bt->i8pre = (const long long*)(base + o_pre);
   for (int k = 0; k < 5; ++k) bt->i8tot[k] = pre[(size_t)k * (nblk + 1) + nblk];

@@ -568,10 +568,13 @@ __device__ __forceinline__ bool brick_origin(const Dims& d, int* ox, int* oy, in
 }
 
 template <class G>
+inline long brick_count(const Dims& d) {
+  return (long)((d.n[0] + G::BX - 1) / G::BX) * ((d.n[1] + G::BY - 1) / G::BY) *
+         ((d.n[2] + G::BZ - 1) / G::BZ);
+}
+template <class G>
 inline unsigned brick_blocks(const Dims& d) {
-  const long nb = (long)((d.n[0] + G::BX - 1) / G::BX) * ((d.n[1] + G::BY - 1) / G::BY) *
-                  ((d.n[2] + G::BZ - 1) / G::BZ);
-  return (unsigned)((nb + 7) & ~7L);
+  return (unsigned)((brick_count<G>(d) + 7) & ~7L);
 }
 
 template <class G>

@@ -63,26 +63,21 @@ void k_fused_group(StageArgs args, Dims d, Scales w, Scal sc) {
   bssn_rhs_point<KO>(src, with_ssl(sc, args.tdev, args.toff), out);
 }
 
-// A grid whose wave-private bricks all fit the chip at once, one per SIMD (4 x 256), is one
-// wave's latency long either way, and the wave-private form's is the shorter (no barriers, more
-// registers): FD4 RK4 step at 24^3 / 32^3 / 40^3 (1000 bricks) 115 / 127 / 155 us against 135 /
-// 141 / 192 us. Past it the shared bricks win: 48^3 (1728) 271 against 213, 64^3 539 against
-// 430, 128^3 4.39 against 3.20 ms.
-// The shared form addresses a field by 32-bit byte offsets, so fields of 4 GiB and more (a state
-// of 103 GB: only the bare RHS fits the card) take the wave-private form too.
-constexpr unsigned kWaveBricks = 4 * 256;
-
+// The shared form where it is the faster one (fused_shared) and its 32-bit byte offsets reach
+// every point: fields of 4 GiB and more (a state of 103 GB: only the bare RHS fits the card) take
+// the wave-private form.
 template <int ORD, bool KO, int MODE, int KIND, bool SDEV>
 static hipError_t launch_fused_t(const StageArgs& a, const Dims& d, const Scales& w,
                                  const Scal& sc, hipStream_t st) {
   using W = Geo<ORD, KO>;
   using G = GroupGeo<ORD, KO>;
-  if (brick_blocks<W>(d) <= kWaveBricks || d.P >= kGroupPoints)
-    hipLaunchKernelGGL((k_fused<ORD, KO, MODE, KIND, SDEV>), dim3(brick_blocks<W>(d)),
-                       dim3(W::NT), 0, st, a, d, w, sc);
-  else
+  if (d.P < kGroupPoints &&
+      fused_shared(ORD, KIND == KIND_RHS, KO, false, brick_count<W>(d), brick_count<G>(d)))
     hipLaunchKernelGGL((k_fused_group<ORD, KO, MODE, KIND, SDEV>), dim3(brick_blocks<G>(d)),
                        dim3(G::NT), 0, st, a, d, w, sc);
+  else
+    hipLaunchKernelGGL((k_fused<ORD, KO, MODE, KIND, SDEV>), dim3(brick_blocks<W>(d)),
+                       dim3(W::NT), 0, st, a, d, w, sc);
   return hipGetLastError();
 }
 

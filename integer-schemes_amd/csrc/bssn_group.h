@@ -46,6 +46,7 @@
 #include <type_traits>
 
 #include "bssn_brick.h"
+#include "bssn_dispatch.h"
 
 namespace bssn {
 
@@ -129,9 +130,6 @@ struct NumeratorTable {
 
 template <class G>
 __constant__ NumeratorTable<G> kNumerators = NumeratorTable<G>();
-
-// Points of a field from which its bytes no longer fit 32-bit offsets (4 GiB).
-constexpr long kGroupPoints = 1L << 29;
 
 // Barrier of the workgroup that orders its LDS accesses (global loads and stores stay in
 // flight across it).

@@ -130,6 +130,29 @@ def test_batched_form_equals_single_grid(sizes, order, waves):
         assert torch.equal(batch.view(U, b), F), b
 
 
+@pytest.mark.parametrize("n", [(64, 66, 8), (48, 47, 56), (63, 64, 20)])
+@pytest.mark.parametrize("order", [4, 6, 8])
+@pytest.mark.parametrize("ko", [0.0, 0.1])
+def test_grids_of_either_form(n, order, ko):
+    """More wave-private bricks than the chip holds, but thin along z or with a last round of
+    shared bricks nearly empty, so that the rule keeps some orders and kinds wave-private: the same
+    bits as persistent waves on wave-private bricks."""
+    print(f"[case] either form {n} order {order} ko {ko}", flush=True)
+    ng = 3 if order == 4 else 4
+    batch = BlockBatch([Block(n=n, h=H3)], ng=ng, device=DEV)
+    batch.set_launch(64)
+    U = batch.empty_pool()
+    batch.view(U, 0).copy_(torch.from_numpy(waves_of(n, ng, order)))
+    F, out = batch.view(U, 0).clone(), torch.empty_like(U)
+    one = torch.empty_like(F)
+    batch.rhs_into(U, out, P, 0.02, order=order, ko_sigma=ko)
+    rhs_into(F, one, scalars(P, *H3, 0.02, 0.0), order, ko)
+    assert torch.equal(batch.view(out, 0), one)
+    batch.step_(U, 0.0, 0.02, P, order=order, ko_sigma=ko, bc="periodic")
+    BSSNEvolution(Grid(*n, *H3, ng=ng), P, order=order, ko_sigma=ko).step_(F, 0.0, 0.02)
+    assert torch.equal(batch.view(U, 0), F)
+
+
 @pytest.mark.parametrize("shape", [(5, 6, 7), (9, 4, 17), (20, 23, 31), (12, 13, 48)])
 @pytest.mark.parametrize("order", [4, 6, 8])
 def test_bundle_maxima_and_constraints(shape, order):
