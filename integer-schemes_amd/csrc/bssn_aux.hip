@@ -479,6 +479,21 @@ struct ConsOut {
   }
 };
 
+// Wave-private bricks, for grids of about one round of them and thin ones (constraints_shared).
+template <int ORD>
+__global__ __launch_bounds__(64) void k_constraints_wave(const double* __restrict__ F,
+                                                         double* __restrict__ HM, Dims d,
+                                                         Scales w) {
+  using G = Geo<ORD, false>;
+  __shared__ double lds[G::VOL];
+  int ox, oy, oz;
+  if (!brick_origin<G>(d, &ox, &oy, &oz)) return;
+  const int lane = (int)threadIdx.x;
+  WaveSrc<ORD, false, CLAMP, ConsOrder> s(lds, F, w, d, ox, oy, oz, lane);
+  ConsOut o{HM, d.P, s.gp, lane_valid<G>(d, ox, oy, oz, lane)};
+  bssn_constraints_point(s, o);
+}
+
 // Bricks shared by four waves, two waves per SIMD (bssn_group.h). Like the fused kernels it waited
 // on memory at one wave per SIMD (376 registers): 150^3 FD4 0.80 -> 0.60 ms.
 template <int ORD, bool WIDE>
@@ -499,8 +514,12 @@ hipError_t launch_constraints(const double* F, double* HM, const Dims& d, const 
                               int ord, hipStream_t st) {
   with_order(ord, [&](auto oc) {
     constexpr int O = decltype(oc)::value;
+    using W = Geo<O, false>;
     using G = GroupGeo<O, false>;
-    if (d.P < kGroupPoints)
+    if (!constraints_shared(O, brick_count<W>(d), brick_count<G>(d)))
+      hipLaunchKernelGGL(k_constraints_wave<O>, dim3(brick_blocks<W>(d)), dim3(W::NT), 0, st, F,
+                         HM, d, w);
+    else if (d.P < kGroupPoints)
       hipLaunchKernelGGL((k_constraints<O, false>), dim3(brick_blocks<G>(d)), dim3(G::NT), 0, st,
                          F, HM, d, w);
     else

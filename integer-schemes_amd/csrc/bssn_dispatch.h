@@ -17,7 +17,8 @@ constexpr long kGroupSlots = 2 * 256;
 
 // Whether `groups` shared bricks take less time than `waves` wave-private bricks over the same
 // points. Both run in rounds of as many as fit the chip; the last round of shared bricks counts
-// 0.7 if it leaves one workgroup per compute unit (measured 0.6 to 0.75). cost: what a full round
+// 0.7 if it leaves one workgroup per compute unit (measured 0.6 to 0.75), and a launch of at most
+// half a round of wave-private ones 0.75 (0.7 to 0.8). cost: what a full round
 // of shared bricks (twice the lanes) takes, in rounds of wave-private ones. Counting rounds and
 // not points covers both ways of wasting a shared brick: lanes without a point (its 16 points
 // along z on a grid of 8) and a last round nearly empty (48 x 48 x 56 is two wave-private rounds
@@ -26,7 +27,8 @@ constexpr bool shared_pays(double cost, long waves, long groups) {
   const long rest = groups % kGroupSlots;
   const double shared =
       (double)(groups / kGroupSlots) + (rest == 0 ? 0.0 : (rest <= kGroupSlots / 2 ? 0.7 : 1.0));
-  return cost * shared <= (double)((waves + kWaveSlots - 1) / kWaveSlots);
+  return cost * shared <=
+         (2 * waves <= kWaveSlots ? 0.75 : (double)((waves + kWaveSlots - 1) / kWaveSlots));
 }
 
 // The fused kernels (a single grid's or a batch's, over the points of one launch). At most one
@@ -51,6 +53,16 @@ constexpr bool fused_shared(int ord, bool rhs, bool ko, bool batch, long waves, 
                       : ord == 6 ? (ko ? 1.19 : 1.11)
                                  : (rhs && ko ? 1.05 : (batch ? 1.03 : 1.0));
   return waves > kWaveSlots && shared_pays(cost, waves, groups);
+}
+
+// The constraints, whose 24^3 and 32^3 samples of long runs are single rounds: FD4 24^3 / 32^3 /
+// 40^3 11.5 / 12.0 / 13.7 us wave-private, 14.7 / 14.7 / 19.3 shared; FD6 15.8 / 16.6 / 19.7 and
+// 17.3 / 17.4 / 23.5; FD8 20.7 / 21.8 / 26.6 and 21.0 / 21.1 / 29.4. Near the line
+// (wave-private / shared time): FD4 39x82x75 1.08, 128x128x24 1.06, 64x64x16 0.95, 103x66x33
+// 0.91, 48x48x56 0.82; FD6 64x64x12 1.07, 160x160x17 1.01, 45x45x52 0.97, 160x160x8 0.89; FD8
+// 72x72x20 1.07, 100x100x8 1.05, 160x160x8 0.97, 256x256x8 0.90.
+constexpr bool constraints_shared(int ord, long waves, long groups) {
+  return shared_pays(ord == 4 ? 1.44 : (ord == 6 ? 1.19 : 1.1), waves, groups);
 }
 
 }  // namespace bssn

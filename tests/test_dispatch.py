@@ -73,3 +73,21 @@ def test_fused_form(tmp_path):
                 want.append(bool(shared))
     got = ask(tmp_path, "fused_shared(ord, what[0] == 'b', what[0] == 's', what[4] == '+', waves, groups)", rows)
     assert got == want, [(r, w) for r, w, g in zip(rows, want, got) if g != w]
+
+
+# (FD4, FD6, FD8) of the constraints
+CONSTRAINTS = [
+    ((12, 12, 12), (0, 0, None)), ((24, 24, 24), (0, 0, None)), ((32, 32, 32), (0, 0, None)),
+    ((40, 40, 40), (0, 0, 0)), ((64, 64, 12), (0, 1, 1)), ((64, 64, 16), (0, 1, 1)),
+    ((48, 48, 48), (1, 1, 1)), ((48, 48, 56), (0, None, 1)), ((103, 66, 33), (0, 1, 1)),
+    ((39, 82, 75), (1, 1, 1)), ((128, 128, 24), (1, 1, 1)), ((160, 160, 8), (0, 0, 0)),
+    ((256, 256, 8), (0, 0, 0)), ((256, 256, 4), (0, 0, 0)), ((150, 150, 150), (1, 1, 1)),
+]
+
+
+def test_constraints_form(tmp_path):
+    rows = [row("c", order, n) for n, faster in CONSTRAINTS
+            for order, shared in zip((4, 6, 8), faster) if shared is not None]
+    want = [bool(v) for _, faster in CONSTRAINTS for v in faster if v is not None]
+    got = ask(tmp_path, "constraints_shared(ord, waves, groups)", rows)
+    assert got == want, [(r, w) for r, w, g in zip(rows, want, got) if g != w]

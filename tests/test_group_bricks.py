@@ -186,3 +186,17 @@ def test_bundle_maxima_and_constraints(shape, order):
     err = normwise(torch.stack([C[k] for k in ("H", "M0", "M1", "M2")]).cpu().numpy(),
                    O.constraints(F, list(H3), order))
     assert err.max() < TOL, err
+
+
+@pytest.mark.parametrize("shape", [(24, 23, 25), (40, 40, 40), (41, 45, 49), (48, 47, 56),
+                                   (70, 72, 8), (33, 130, 16)])
+@pytest.mark.parametrize("order", [4, 6, 8])
+def test_constraints_of_either_form(shape, order):
+    """The constraints on both sides of the rule that picks their form."""
+    print(f"[case] constraints {shape} order {order}", flush=True)
+    F = waves(shape, seed=order)
+    grid = Grid(*[n - 4 for n in shape], *H3, ng=order // 2)
+    C = ConstraintSolver(grid, order=order).constraints(torch.from_numpy(F).to(DEV))
+    err = normwise(torch.stack([C[k] for k in ("H", "M0", "M1", "M2")]).cpu().numpy(),
+                   O.constraints(F, list(H3), order))
+    assert err.max() < TOL, err
