@@ -91,18 +91,18 @@ __device__ __forceinline__ void bundle_put(const BundleOut& o, int slot, long P,
   }
 }
 
-// Bricks shared by four waves (bssn_group.h), kFieldRun fields per
-// workgroup (blockIdx.y). What bounds the pass is the store of the 138 arrays (with the stencils
-// left out it takes as long): 4 x 4 x 16 bricks write rows of 128 B, where a wave's own 4 x 4 x 4
-// brick wrote pieces of 32 B, and the runs, dispatched one after the other, write 3 to 18 arrays
-// at a time instead of 138. 134^3, FD6 fp64 / 118^3, FD4 BFP32: 2.08 / 0.96 -> 1.33 / 0.50 ms (runs
-// of 1 / 3 / 4 / 8 / 24 fields: 1.38 / 1.35 / 1.37 / 1.43 / 1.48 and 0.53 / 0.50 / 0.51 / 0.51 /
-// 0.54); with the shared numerators FD6 1.29, 134^3 FD4 fp64 1.25 -> 1.14 ms. Rows that start on a 128 B line write a quarter faster (2.85 against 2.13 TB/s); the
-// caller's row pitch decides that.
+// Bricks shared by four waves (bssn_group.h), kFieldRun fields per workgroup (blockIdx.y). What
+// bounds the pass is the store of the 138 arrays (with the stencils left out it takes as long):
+// 4 x 4 x 16 bricks write rows of 128 B, where a wave's own 4 x 4 x 4 brick wrote pieces of 32 B,
+// and the runs, dispatched one after the other, write 3 to 18 arrays at a time instead of 138.
+// 134^3, FD6 fp64 / 118^3, FD4 BFP32: 2.08 / 0.96 -> 1.33 / 0.50 ms (runs of 1 / 3 / 4 / 8 / 24
+// fields: 1.38 / 1.35 / 1.37 / 1.43 / 1.48 and 0.53 / 0.50 / 0.51 / 0.51 / 0.54); with the shared
+// numerators FD6 1.29, 134^3 FD4 fp64 1.25 -> 1.14 ms. Rows that start on a 128 B line write a
+// quarter faster (2.85 against 2.13 TB/s).
 constexpr int kFieldRun = 2;
 static_assert(BSSN_NF % kFieldRun == 0, "whole runs");
 
-template <int ORD, int STORE, bool WIDE>
+template <int ORD, int STORE>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(ORD == 8 ? 2 : 4)))
 void k_deriv_bundle(const double* __restrict__ F, BundleOut o, Dims d, Scales w) {
@@ -112,7 +112,7 @@ void k_deriv_bundle(const double* __restrict__ F, BundleOut o, Dims d, Scales w)
   if (!brick_origin<G>(d, &ox, &oy, &oz)) return;
   const int t = (int)threadIdx.x, f0 = (int)blockIdx.y * kFieldRun;
   const bool valid = lane_valid<G>(d, ox, oy, oz, t);
-  GroupSrc<ORD, false, CLAMP, StateOrder, WIDE> s(mem, F, w, d, ox, oy, oz, t, f0);
+  GroupSrc<ORD, false, CLAMP, StateOrder> s(mem, F, w, d, ox, oy, oz, t, f0);
 #pragma unroll 1
   for (int i = 0; i < kFieldRun; ++i) {
     const int f = f0 + i, sl = s2slot(f);
@@ -127,17 +127,57 @@ void k_deriv_bundle(const double* __restrict__ F, BundleOut o, Dims d, Scales w)
   }
 }
 
+// Wave-private bricks, all fields by one wave: arrays thin along z (bundle_shared), and fields of
+// 4 GiB and more, past the shared form's byte offsets. FD4 fp64 and BFP32 stores: two fields in
+// flight, stepped in pairs so each staging slot is a constant (256^3: two-pass RHS with KO 28.6 ->
+// 26.8 ms, BFP32 15.9 -> 13.1 ms); the others keep one (BFP48 19.0 -> 21.1 ms with two).
+template <int ORD, int STORE>
+__global__ __launch_bounds__(64) void k_deriv_bundle_wave(const double* __restrict__ F,
+                                                          BundleOut o, Dims d, Scales w) {
+  using G = Geo<ORD, false>;
+  __shared__ double lds[G::VOL];
+  int ox, oy, oz;
+  if (!brick_origin<G>(d, &ox, &oy, &oz)) return;
+  const int lane = (int)threadIdx.x;
+  const bool valid = lane_valid<G>(d, ox, oy, oz, lane);
+  constexpr int DEPTH = ORD == 4 && STORE != BS_Q48 ? 2 : 1;
+  WaveSrc<ORD, false, CLAMP, StateOrder, DEPTH> s(lds, F, w, d, ox, oy, oz, lane);
+  for_fields<DEPTH>([&](int f, auto slot) {
+    s.template stage_slot<decltype(slot)::value>(f);
+    double v[9];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) v[a] = s.d1(a);
+    const int sl = s2slot(f);
+    if (sl >= 0) {
+#pragma unroll
+      for (int q = 0; q < 6; ++q) v[3 + q] = s.d2(pi_(q), pj_(q));
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) bundle_put<STORE>(o, 3 * f + a, d.P, s.gp, v[a], valid);
+    if (sl >= 0) {
+#pragma unroll
+      for (int q = 0; q < 6; ++q)
+        bundle_put<STORE>(o, 72 + 6 * sl + q, d.P, s.gp, v[3 + q], valid);
+    }
+    __builtin_amdgcn_wave_barrier();
+  });
+}
+
 template <int STORE>
 static void launch_bundle_store(const double* F, const BundleOut& o, const Dims& d,
                                 const Scales& w, int ord, hipStream_t st) {
   with_order(ord, [&](auto oc) {
     constexpr int O = decltype(oc)::value;
+    using W = Geo<O, false>;
     using G = GroupGeo<O, false>;
-    const dim3 grid(brick_blocks<G>(d), BSSN_NF / kFieldRun);
-    if (d.P < kGroupPoints)
-      hipLaunchKernelGGL((k_deriv_bundle<O, STORE, false>), grid, dim3(G::NT), 0, st, F, o, d, w);
+    if (d.P < kGroupPoints &&
+        bundle_shared(O, STORE == BS_F64, brick_count<W>(d), brick_count<G>(d)))
+      hipLaunchKernelGGL((k_deriv_bundle<O, STORE>),
+                         dim3(brick_blocks<G>(d), BSSN_NF / kFieldRun), dim3(G::NT), 0, st, F, o,
+                         d, w);
     else
-      hipLaunchKernelGGL((k_deriv_bundle<O, STORE, true>), grid, dim3(G::NT), 0, st, F, o, d, w);
+      hipLaunchKernelGGL((k_deriv_bundle_wave<O, STORE>), dim3(brick_blocks<W>(d)), dim3(W::NT),
+                         0, st, F, o, d, w);
   });
 }
 

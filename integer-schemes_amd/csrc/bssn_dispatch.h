@@ -65,4 +65,16 @@ constexpr bool constraints_shared(int ord, long waves, long groups) {
   return shared_pays(ord == 4 ? 1.44 : (ord == 6 ? 1.19 : 1.1), waves, groups);
 }
 
+// The derivative bundle. The shared bricks write longer rows and few arrays at a time, so they win
+// at every size (12^3 FD4 18.0 -> 5.8 us) unless half of their lanes or more have no point: arrays
+// of up to 8 points along z, of more than one round of wave-private bricks at FD4, of two above.
+// (wave-private / shared, FD4 fp64, BFP32 and FD6 fp64, BFP32): 256x256x8 1.09, 0.68, 0.90, 0.73;
+// 160x160x8 1.16, 0.61, 0.92, 0.92; 100x100x8 0.90, 0.92, 1.10, 1.11; 256x256x4 0.53, 0.28, 0.51,
+// 0.39; 160x160x17 1.48, 1.14, 1.41, 0.96. The maxima are faster shared at every size but of four
+// points along z above FD4 (256x256x4 FD6 0.86, 160x160x8 1.58), narrower than their stencils.
+constexpr bool bundle_shared(int ord, bool fp64, long waves, long groups) {
+  if (ord == 4 && fp64) return groups < waves || waves <= kWaveSlots;
+  return 2 * groups < waves || waves <= (ord == 4 ? 1 : 2) * kWaveSlots;
+}
+
 }  // namespace bssn

@@ -91,3 +91,23 @@ def test_constraints_form(tmp_path):
     want = [bool(v) for _, faster in CONSTRAINTS for v in faster if v is not None]
     got = ask(tmp_path, "constraints_shared(ord, waves, groups)", rows)
     assert got == want, [(r, w) for r, w, g in zip(rows, want, got) if g != w]
+
+
+# (FD4 fp64, FD4 BFP32, FD6 fp64, FD6 BFP32) of the derivative bundle
+BUNDLE = [
+    ((12, 12, 12), (1, 1, 1, 1)), ((40, 40, 40), (1, 1, 1, 1)), ((128, 128, 128), (1, 1, 1, 1)),
+    ((72, 72, 8), (1, 1, 1, 1)), ((100, 100, 8), (None, 0, 1, 1)), ((160, 160, 8), (1, 0, 0, 0)),
+    ((256, 256, 8), (1, 0, 0, 0)), ((256, 256, 4), (0, 0, 0, 0)), ((200, 200, 20), (1, 1, 1, 1)),
+    ((96, 96, 12), (1, 1, 1, 1)),
+]
+
+
+def test_bundle_form(tmp_path):
+    rows, want = [], []
+    for n, faster in BUNDLE:
+        for i, shared in enumerate(faster):
+            if shared is not None:
+                rows.append(row(("fp64", "bfp")[i % 2], (4, 6)[i // 2], n))
+                want.append(bool(shared))
+    got = ask(tmp_path, "bundle_shared(ord, what[0] == 'f', waves, groups)", rows)
+    assert got == want, [(r, w) for r, w, g in zip(rows, want, got) if g != w]

@@ -10,6 +10,8 @@ rates they enter; every other term is smaller.
 """
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -22,7 +24,7 @@ from bssn3d_hip.batch import Block, BlockBatch
 from bssn3d_hip.constraints import ConstraintSolver
 from bssn3d_hip.evolve import BSSNEvolution
 from bssn3d_hip.grid import Grid
-from bssn3d_hip.rhs import rhs_into, stream_handle
+from bssn3d_hip.rhs import bfp_buffers, rhs_into, stream_handle
 from bssn3d_hip.state import PhysicsParams, scalars
 
 pytestmark = [pytest.mark.gpu,
@@ -200,3 +202,41 @@ def test_constraints_of_either_form(shape, order):
     err = normwise(torch.stack([C[k] for k in ("H", "M0", "M1", "M2")]).cpu().numpy(),
                    O.constraints(F, list(H3), order))
     assert err.max() < TOL, err
+
+
+@pytest.mark.parametrize("shape", [(150, 90, 7), (290, 130, 4), (41, 45, 49)])
+@pytest.mark.parametrize("order", [4, 6, 8])
+def test_bundle_of_either_form(shape, order):
+    """The bundle thin along z (wave-private bricks) and not, in each storage, against the oracle's
+    with the bound of a derivative's rounding error above. The maxima, which have one form, are
+    those of the stored bundle exactly, over more bricks than they have workgroups; BFP storage
+    holds the fp64 bundle's values at 2^-e."""
+    print(f"[case] bundle {shape} order {order}", flush=True)
+    F = waves(shape, seed=order)
+    Fd = torch.from_numpy(F).to(DEV)
+    D = torch.empty((138,) + tuple(shape), dtype=torch.float64, device=DEV)
+    amax = torch.empty(138, dtype=torch.float64, device=DEV)
+    lib, st, h3 = _lib.load(), stream_handle(Fd.device), _lib.dbl(H3)
+    _lib.check(lib.bssn_deriv_bundle_f64(Fd.data_ptr(), D.data_ptr(), *shape, order, h3, st))
+    _lib.check(lib.bssn_deriv_bundle_absmax_f64(Fd.data_ptr(), amax.data_ptr(), *shape, order,
+                                                h3, st))
+    assert torch.equal(amax, D.abs().flatten(1).max(dim=1).values)
+    got, ref = D.cpu().numpy(), O.deriv_bundle(F, list(H3), order)
+    c1, c2 = (np.abs(O.stencil(k, order)).sum() for k in (0, 1))
+    for d in range(138):
+        if d < 72:
+            f, a = divmod(d, 3)
+            mag = c1 / H3[a]
+        else:
+            s, q = divmod(d - 72, 6)
+            f = O.IDX[O.S2_FIELDS[s]]
+            i, j = O.PAIRS[q]
+            mag = c2 / H3[i] ** 2 if i == j else c1 * c1 / (H3[i] * H3[j])
+        assert np.abs(got[d] - ref[d]).max() <= 64 * 2.2e-16 * mag * np.abs(F[f]).max(), d
+    e = [int(v) for v in 24 - np.frexp(amax.cpu().numpy())[1]]
+    Q, _ = bfp_buffers(Fd, 32)
+    _lib.check(lib.bssn_deriv_bundle_bfp(Fd.data_ptr(), Q.data_ptr(), (ctypes.c_int * 138)(*e), 32,
+                                         *shape, order, h3, st))
+    scale = torch.tensor([2.0 ** v for v in e], dtype=torch.float64, device=DEV)
+    stored = Q[Q.numel() - 4 * D.numel():].view(torch.int32).view(D.shape)   # after the header
+    assert torch.equal(stored.double(), torch.round(D * scale.view(-1, 1, 1, 1)))
