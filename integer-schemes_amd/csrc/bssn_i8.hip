@@ -13,7 +13,8 @@
 //   box values v -> c = 0.5 max + 0.5 min (stencils annihilate constants), sigma = 2^(6-E) with
 //   max|v - c| = f 2^E, r0 = (v - c) sigma, q_s = rint(r_s), r_{s+1} = 128 (r_s - q_s):
 //   |q_s| <= 64, every step exact; (v - c) sigma = sum_s q_s 2^(-7 s) + O(2^(-7 k)).
-//   The k <= 7 digits are taken in three groups (0..2, 3..5, 6), each as one integer
+//   The k <= 7 digits are taken in groups of three (0..2, 3..5, and the last by itself where that
+//   leaves one), each as one integer
 //   N = rint(r 2^(7 (g - 1))) = sum_s q_s 2^(7 (g - 1 - s)) (g digits; the remainder is the same,
 //   and a tie falls the same way), whose signed bytes are the int8 operands (32 x 32 planes):
 //     B N   (rows: outputs along axis 1)   = sum of v_mfma_i32_32x32x32_i8(band, byte plane)
@@ -171,9 +172,11 @@ __host__ __device__ inline long i8_tiles(const int* S) {
 }
 
 // ORIENT 0: (y, z) planes at each x; 1: (x, z) planes at each y; 2: (x, y) planes at each z.
-// TWO: the fields with second derivatives (else first derivatives only).
-// One wave: tile w (plane fastest, then tile along axis 2, along axis 1, field) of the grid a.
-template <int ORIENT, bool TWO>
+// TWO: the fields with second derivatives (else first derivatives only). ONE: a single digit,
+// which as a group of three is multiplied as three byte planes (16^3 / 64^3: 40.5 / 176 -> 35.3 /
+// 139 us, the same in one plane).
+// One wave: tile w of the grid a, in the order below.
+template <int ORIENT, bool TWO, bool ONE>
 __device__ __forceinline__ void i8_tile(const I8Args& a, long w, int lane, int* t) {
   constexpr int AX1 = ORIENT == 0 ? 1 : 0;
   constexpr int AX2 = ORIENT == 2 ? 1 : 2;
@@ -250,9 +253,10 @@ __device__ __forceinline__ void i8_tile(const I8Args& a, long w, int lane, int* 
     for (int j = 0; j < 16; ++j) r[j] = r[j] == INFINITY ? -1.0 : 0.0;
   }
 
-  // digits 0..na-1, na..na+nb-1 and 6
+  // the groups of ns digits: 0..na-1 (ONE: none), 3..nb+2 (from five), and the last digit by
+  // itself where threes leave one
   const int ns = a.nslice, na = ns < 3 ? ns : 3, nb = ns < 6 ? ns - na : 3;
-  const bool more = ns > 3, last = ns > 6;
+  const bool more = !ONE && ns > 4, last = ONE || ns % 3 == 1;
   v4i qa[3], qb[3], qc[1], ta[3], tb[3], tc[1];   // byte planes of N and of N^T
   constexpr bool COLS = D1B || D2B;
   auto digits = [&](auto np, int g, v4i* q, v4i* tr) {
@@ -273,11 +277,11 @@ __device__ __forceinline__ void i8_tile(const I8Args& a, long w, int lane, int* 
       row_planes<NP>(t, lane, tr);
     }
   };
-  digits(std::integral_constant<int, 3>(), na, qa, ta);
+  if constexpr (!ONE) digits(std::integral_constant<int, 3>(), na, qa, ta);
   if (more) digits(std::integral_constant<int, 3>(), nb, qb, tb);
   if (last) digits(std::integral_constant<int, 1>(), 1, qc, tc);
   const double wa = ldexp(1.0, -7 * (na - 1)), wb = ldexp(1.0, -7 * (na + nb - 1)),
-               wc = ldexp(1.0, -42);
+               wc = ldexp(1.0, -7 * (ns - 1));
   double acc[16];
   auto add = [&](const v16i& p, double ws) {
 #pragma unroll
@@ -309,7 +313,7 @@ __device__ __forceinline__ void i8_tile(const I8Args& a, long w, int lane, int* 
   const int slot = TWO ? fi : -1;
   auto columns = [&](const v4i& band) {
     clear();
-    add(contract<3, false>(band, ta), wa);
+    if constexpr (!ONE) add(contract<3, false>(band, ta), wa);
     if (more) add(contract<3, false>(band, tb), wb);
     if (last) add(contract<1, false>(band, tc), wc);
   };
@@ -323,7 +327,7 @@ __device__ __forceinline__ void i8_tile(const I8Args& a, long w, int lane, int* 
   }
   auto rows = [&](const v4i& band) {
     clear();
-    add(contract<3, true>(band, qa), wa);
+    if constexpr (!ONE) add(contract<3, true>(band, qa), wa);
     if (more) add(contract<3, true>(band, qb), wb);
     if (last) add(contract<1, true>(band, qc), wc);
   };
@@ -348,7 +352,7 @@ __device__ __forceinline__ void i8_tile(const I8Args& a, long w, int lane, int* 
       add(contract<NP, false>(band1, pl), ws);
     };
     clear();
-    mixed(std::integral_constant<int, 4>(), contract<3, true>(band1, qa), wa);
+    if constexpr (!ONE) mixed(std::integral_constant<int, 4>(), contract<3, true>(band1, qa), wa);
     if (more) mixed(std::integral_constant<int, 4>(), contract<3, true>(band1, qb), wb);
     if (last) mixed(std::integral_constant<int, 2>(), contract<1, true>(band1, qc), wc);
     // pair index of (AX1, AX2): xy 1, xz 2, yz 4; scale index AX1 + AX2 - 1
@@ -379,19 +383,19 @@ __device__ __forceinline__ long xcd_tile() {
 // 0.34 -> 0.31, (x, y) planes 0.64 ms. Three or four waves per SIMD spill where second derivatives
 // are taken (0.70 -> 0.85 and 1.11 ms); the first-derivative pass on (x, z) planes has the room
 // for four (0.31 -> 0.26 ms).
-template <int ORIENT, bool TWO>
+template <int ORIENT, bool TWO, bool ONE>
 __global__ __launch_bounds__(64)
 __attribute__((amdgpu_waves_per_eu(ORIENT == 1 && !TWO ? 4 : 1)))
 void k_i8_plane(I8Args a) {
   BSSN_I8_LDS;
-  i8_tile<ORIENT, TWO>(a, xcd_tile(), (int)threadIdx.x, t);
+  i8_tile<ORIENT, TWO, ONE>(a, xcd_tile(), (int)threadIdx.x, t);
 }
 
 // The same pass over every block of a batch: block b owns wave tiles [pre[b], pre[b + 1]) of
 // the launch; its bundle is the 138 arrays at D + blk[b].doff and its stencil scales are formed
 // from its spacings with the host's rounding, so each block's bundle equals the single-grid
 // bundle of that block bit for bit.
-template <int ORIENT, bool TWO>
+template <int ORIENT, bool TWO, bool ONE>
 __global__ __launch_bounds__(64) void k_i8_plane_batch(const double* pool, double* D,
                                                        const BlockDesc* __restrict__ blks,
                                                        const long long* __restrict__ pre,
@@ -418,14 +422,17 @@ __global__ __launch_bounds__(64) void k_i8_plane_batch(const double* pool, doubl
     a.sm[i] = uniform(sc.sm[i]);
   }
   a.nslice = nslice;
-  i8_tile<ORIENT, TWO>(a, (long)(w - pre[b]), (int)threadIdx.x, t);
+  i8_tile<ORIENT, TWO, ONE>(a, (long)(w - pre[b]), (int)threadIdx.x, t);
 }
 
 template <int ORIENT, bool TWO>
 static hipError_t launch_i8_t(const I8Args& a, hipStream_t st) {
   const long n = (i8_tiles<ORIENT, TWO>(a.S) + 7) & ~7L;
   if (n > 0x7fffffffL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_i8_plane<ORIENT, TWO>), dim3((unsigned)n), dim3(64), 0, st, a);
+  if (a.nslice == 1)
+    hipLaunchKernelGGL((k_i8_plane<ORIENT, TWO, true>), dim3((unsigned)n), dim3(64), 0, st, a);
+  else
+    hipLaunchKernelGGL((k_i8_plane<ORIENT, TWO, false>), dim3((unsigned)n), dim3(64), 0, st, a);
   return hipGetLastError();
 }
 
@@ -448,8 +455,12 @@ static hipError_t launch_i8_batch_t(const double* pool, double* D, const BlockDe
   if (n == 0) return hipSuccess;
   n = (n + 7) & ~7LL;
   if (n > 0x7fffffffLL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_i8_plane_batch<ORIENT, TWO>), dim3((unsigned)n), dim3(64), 0, st, pool,
-                     D, blk, pre, nblk, nslice);
+  if (nslice == 1)
+    hipLaunchKernelGGL((k_i8_plane_batch<ORIENT, TWO, true>), dim3((unsigned)n), dim3(64), 0, st,
+                       pool, D, blk, pre, nblk, nslice);
+  else
+    hipLaunchKernelGGL((k_i8_plane_batch<ORIENT, TWO, false>), dim3((unsigned)n), dim3(64), 0, st,
+                       pool, D, blk, pre, nblk, nslice);
   return hipGetLastError();
 }
 
