@@ -146,6 +146,37 @@ def test_prolong_blocks_bitwise(BS, ng):
         assert np.all(blk[:, ~mask] == -7.0), (c, sk)
 
 
+@pytest.mark.parametrize("BS,ng", [(8, 3), (10, 2), (12, 3), (16, 4), (18, 3)])
+def test_prolong_blocks_with_supplied_z_faces(BS, ng):
+    """Jobs whose z faces come from neighbours: planes inside the block form their 2 ng ghost rows
+    only. With and without the other faces and the interior, for slabs that divide the padded
+    extent and slabs that do not."""
+    say(f"block prolongation without z faces, BS={BS} ng={ng}")
+    from amr_emul import job_points
+    from bssn3d_hip.amr import block_job
+    W = BS + 2 * ng
+    P = 24 * W ** 3
+    parent = np.random.default_rng(BS + 2).standard_normal((24, W, W, W))
+    skips = [0b110000, 0b110101, 0b111111, 0b111111 | 64]
+    jobs = [(c, sk) for c in CORNERS for sk in skips]
+    pool = torch.full(((len(jobs) + 1) * P,), -7.0, dtype=torch.float64, device=DEV)
+    pool[:P] = torch.from_numpy(parent.reshape(-1)).to(DEV)
+    e = np.concatenate([block_job((i + 1) * P, 0, c, BS, ng, sk) for i, (c, sk) in
+                        enumerate(jobs)])
+    d = torch.from_numpy(e.view(np.uint8).copy()).to(DEV)
+    _lib.check(_lib.load().bssn_prolong_blocks_f64(pool.data_ptr(), pool.numel(), d.data_ptr(),
+                                                   len(e), stream_handle(pool.device)))
+    got = pool.cpu().numpy()
+    for i, (c, sk) in enumerate(jobs):
+        blk = got[(i + 1) * P:(i + 2) * P].reshape(24, W, W, W)
+        want = OA.prolongate(parent, c, BS, ng)
+        pts = job_points(e[i])
+        mask = np.zeros((W, W, W), bool)
+        mask[pts[:, 0], pts[:, 1], pts[:, 2]] = True
+        assert np.array_equal(blk[:, mask], want[:, mask]), (c, sk)
+        assert np.all(blk[:, ~mask] == -7.0), (c, sk)
+
+
 def test_indicator_bitwise():
     say("indicator")
     H = three_level()
@@ -324,6 +355,26 @@ def test_linked_step_equals_program_step(BS, ng):
     b = host_blocks(H, B)
     for k in H.keys:
         assert np.array_equal(a[k], b[k]), k
+
+
+@pytest.mark.parametrize("BS,ng,order", [(12, 3, 4), (16, 3, 4), (16, 4, 6), (16, 4, 8)])
+def test_linked_step_on_either_form(BS, ng, order):
+    """Linked steps on the bricks the rule picks (shared by four waves for 21 blocks of 16^3, 1344
+    wave-private bricks; wave-private for 12^3, 567) and on persistent wave-private ones: the same
+    bits."""
+    say(f"linked steps on either form, BS={BS}, ng={ng}, order {order}")
+    H = three_level(BS, ng)
+    bricks = len(H.keys) * (BS // 4) ** 3
+    assert (bricks > 1024) == (BS == 16)
+    A = H.fill(H.empty_pool(), smooth_fn(11))
+    B = A.clone()
+    p, dt = PhysicsParams(), 0.25 * H.spacing(2)
+    H.step_(A, 0.1, dt, p, order=order, ko_sigma=0.1, ghosts="linked")
+    H.batch.set_launch(64)
+    H.step_(B, 0.1, dt, p, order=order, ko_sigma=0.1, ghosts="linked")
+    a, b = host_blocks(H, A), host_blocks(H, B)
+    for k in H.keys:
+        assert np.isfinite(a[k]).all() and np.array_equal(a[k], b[k]), k
 
 
 def bump_fn(center=(0.2, 0.2, 0.2), width=0.08, amp=0.05):

@@ -155,6 +155,30 @@ def test_grids_of_either_form(n, order, ko):
     assert torch.equal(batch.view(U, 0), F)
 
 
+@pytest.mark.parametrize("sizes", [[(16, 16, 8)] * 80, [(9, 9, 13)] * 60,
+                                   [(12, 12, 20), (8, 16, 6), (16, 7, 24)] * 14])
+@pytest.mark.parametrize("order", [4, 6, 8])
+def test_batches_of_either_form(sizes, order):
+    """Batches whose blocks leave much of a brick empty, along z (where the rule keeps some orders
+    wave-private) or along x and y: the same bits as persistent waves on wave-private bricks."""
+    print(f"[case] batch form {sizes[:3]} x {len(sizes)} order {order}", flush=True)
+    ng = 3 if order == 4 else 4
+    assert sum(bricks(n) for n in sizes) > 1024
+    batch = BlockBatch([Block(n=n, h=H3) for n in sizes], ng=ng, device=DEV)
+    A = batch.empty_pool()
+    for b, n in enumerate(sizes):
+        batch.view(A, b).copy_(torch.from_numpy(waves_of(n, ng, b % 5)))
+    B, outs = A.clone(), []
+    for U, launch in ((A, 0), (B, 64)):
+        batch.set_launch(launch)
+        outs.append(torch.zeros_like(U))
+        batch.rhs_into(U, outs[-1], P, 0.02, order=order, ko_sigma=0.1)
+        batch.step_(U, 0.0, 0.02, P, order=order, ko_sigma=0.1, bc="periodic")
+    for b in range(len(sizes)):
+        assert torch.equal(batch.view(outs[0], b), batch.view(outs[1], b)), b
+        assert torch.equal(batch.view(A, b), batch.view(B, b)), b
+
+
 @pytest.mark.parametrize("shape", [(5, 6, 7), (9, 4, 17), (20, 23, 31), (12, 13, 48)])
 @pytest.mark.parametrize("order", [4, 6, 8])
 def test_bundle_maxima_and_constraints(shape, order):
