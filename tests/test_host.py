@@ -266,3 +266,41 @@ def test_autotune_space_and_installed_choice():
     assert m["candidates"]["default"]["step_ms"] == 39.5 and m["best"] == "e"
     with pytest.raises(ValueError):
         at.merge(dict(rec, workload="other"), new)
+
+
+def test_autotune_times_and_checks_the_kernels_its_knobs_reach():
+    """The wave-private kernels run grids of at most 1024 bricks: the tuner's small grid is one for
+    every brick shape it tries, inside and with its ghosts, it is checked and timed for every
+    candidate, and only candidates with a knob that the shared bricks read are timed on the large
+    one. A time that a candidate does not have takes no part in the choice."""
+    pkg = ROOT / "integer-schemes_amd"
+    at = _load_module("bssn_autotune", pkg / "autotune.py")
+    rule = (pkg / "csrc" / "bssn_dispatch.h").read_text()
+    slots = [int(a) * int(b) for a, b in re.findall(r"kWaveSlots = (\d+) \* (\d+)", rule)][0]
+    for d in at.SPACES["full"]:
+        e = [d.get(f"BSSN_BRICK_{a}", 4) for a in "XYZ"]
+        for n in (at.SMALL, at.SMALL + 2 * 3):
+            assert int(np.prod([-(-n // v) for v in e])) <= slots, (d, n)
+    assert at.SMALL in at.CHECKS and any(-(-n // 4) ** 3 > slots for n in at.CHECKS)
+    # the knobs that the shared bricks read
+    shared = (pkg / "csrc" / "bssn_group.h").read_text()
+    for d in at.SPACES["full"]:
+        assert "small" in at.timed_on(d)
+        assert ("bench" in at.timed_on(d)) == (not d or "BSSN_BRICK_TILE_XY" in d)
+        assert not [k for k in d if k in shared]
+    base = {"passed": True, "defines": {}, "step_ms": 25.0, "rhs_ms": 4.5, "small_step_ms": 0.11,
+            "small_rhs_ms": 0.02}
+    wave = {"passed": True, "defines": {"BSSN_WB_LEAD": 1}, "small_step_ms": 0.10,
+            "small_rhs_ms": 0.02}
+    order = dict(base, defines={"BSSN_BRICK_TILE_XY": 2}, step_ms=24.0, small_step_ms=0.112)
+    assert at.choose({"default": base, "a": wave, "b": order})["best"] == "a"   # b: slower small
+    assert at.choose({"default": base, "a": dict(wave, passed=False)})["best"] == "default"
+    assert at.choose({"default": base, "a": dict(wave, small_rhs_ms=0.021)})["best"] == "default"
+    assert at.choose({"default": base, "b": dict(order, small_step_ms=0.11)})["best"] == "b"
+    # the installed record was measured on both workloads
+    t = json.loads((pkg / "tuning.json").read_text())
+    assert t["small"] == at.SMALL
+    for k, r in t["candidates"].items():
+        want = {x for w in at.timed_on(r["defines"]) for x in at.TIMES
+                if x.startswith("small_") == (w == "small")}
+        assert want <= set(r), k
